@@ -554,7 +554,7 @@ def main():
             "n_qubits": n, "gates": gates, "method": best,
         },
         "methods": results,
-        # against the faster of the two plain methods (persistent loop, one launch per primitive)
+        # against the faster of the two plain methods (resident rows, one launch per primitive)
         "speedup_vs_plain": (r["gate_updates_per_s"] / max(results[k]["gate_updates_per_s"]
                                                            for k in ("plain", "plain_launch")
                                                            if k in results)

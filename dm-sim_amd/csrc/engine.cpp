@@ -14,6 +14,7 @@
 #include "noalloc.hpp"
 #include "fused.hpp"
 #include "mlp.hpp"
+#include "rows.hpp"
 #include "sweep.hpp"
 
 namespace dmx {
@@ -44,6 +45,7 @@ Engine::~Engine()
     if (d_im2_) (void)hipFree(d_im2_);
     if (d_diag_) (void)hipFree(d_diag_);
     if (d_ops_) (void)hipFree(d_ops_);
+    if (d_rows_) (void)hipFree(d_rows_);
     if (d_probe_blk_) (void)hipFree(d_probe_blk_);
     if (d_probe_blk5_) (void)hipFree(d_probe_blk5_);
     if (d_probe_op_) (void)hipFree(d_probe_op_);
@@ -71,7 +73,6 @@ int Engine::init(uint32_t n_qubits, uint32_t n_gpus)
     HIPTRY(hipMalloc(&d_re_, num_ * sizeof(double)));
     HIPTRY(hipMalloc(&d_im_, num_ * sizeof(double)));
     HIPTRY(hipMalloc(&d_diag_, dim_ * sizeof(double)));
-    HIPTRY(plain_persistent_grid(n_, &persistent_blocks_));
     void* scratch = nullptr;  // the allocation-free gather's staging on this device
     HIPTRY(noalloc_scratch(&scratch));
     return reset_dm();
@@ -137,6 +138,7 @@ int Engine::upload()
         return DMX_ESTATE;
     }
     prims_.clear();
+    row_first_.clear();
     bool wide = false;
     for (const Gate& g : circuit_)
         if (!lower_gate(g, prims_)) wide = true;
@@ -228,6 +230,10 @@ int Engine::upload()
             return DMX_ESTATE;
         }
     }
+    if (!plan_ && method_ != DMX_METHOD_PLAIN_LAUNCH && n_ <= kRowsMaxQubits) {
+        const int rc = ensure_rows();
+        if (rc) return rc;
+    }
     HIPTRY(hipStreamSynchronize(stream_));
     uploaded_ = true;
     return DMX_OK;
@@ -257,7 +263,7 @@ int Engine::run()
         return DMX_ESTATE;
     }
     const int rc = method_ == DMX_METHOD_FUSED && plan_ ? run_fused()
-                                                        : run_plain(method_ != DMX_METHOD_PLAIN);
+                                                        : run_plain(method_ == DMX_METHOD_PLAIN_LAUNCH);
     if (rc == DMX_OK && report_) {
         // the reference's per-run report (src/dmsim_amdgpu_omp.hpp:498-503,
         // on by default through PRINT_MEA_PER_CIRCUIT); one GPU: no
@@ -275,9 +281,37 @@ int Engine::run()
 
 uint64_t Engine::device_bytes() const
 {
-    uint64_t b = 2 * num_ * sizeof(double) + dim_ * sizeof(double) + d_ops_cap_ * sizeof(PrimOp);
+    uint64_t b = 2 * num_ * sizeof(double) + dim_ * sizeof(double) + d_ops_cap_ * sizeof(PrimOp) +
+                 d_rows_cap_ * sizeof(RowOp);
     if (d_re2_) b += 2 * num_ * sizeof(double);
     return b;
+}
+
+int Engine::ensure_rows()
+{
+    if (!row_first_.empty() || prims_.empty()) return DMX_OK;
+    std::vector<RowOp> prog;
+    std::vector<size_t> first;
+    size_t s0 = 0;
+    while (s0 < prims_.size()) {
+        size_t s1 = s0;
+        while (s1 < prims_.size() && prims_[s1].kind != PK_SUP) s1++;
+        if (s1 > s0) first.push_back(build_row_program(prims_, s0, s1, n_, prog));
+        s0 = s1 + 2;
+    }
+    if (first.empty()) return DMX_OK;  // channels only
+    if (prog.size() > d_rows_cap_) {
+        if (d_rows_) HIPTRY(hipFree(d_rows_));
+        d_rows_ = nullptr;
+        d_rows_cap_ = 0;
+        HIPTRY(hipMalloc(&d_rows_, prog.size() * sizeof(RowOp)));
+        d_rows_cap_ = prog.size();
+    }
+    HIPTRY(hipMemcpyAsync(d_rows_, prog.data(), prog.size() * sizeof(RowOp), hipMemcpyHostToDevice,
+                          stream_));
+    HIPTRY(hipStreamSynchronize(stream_));  // the source ends with this call
+    row_first_ = std::move(first);
+    return DMX_OK;
 }
 
 int Engine::run_plain(bool per_launch)
@@ -285,64 +319,56 @@ int Engine::run_plain(bool per_launch)
     const int n_ops = (int)prims_.size();
     last_launches_ = 0;
     last_sweeps_ = 0;
-    last_fallbacks_ = 0;
-    bool coop_ok = true;  // until a cooperative launch of this run is refused
+    const bool rows = !per_launch && n_ <= kRowsMaxQubits;
+    if (rows) {
+        const int rc = ensure_rows();
+        if (rc) return rc;
+    }
     prof_.start(stream_);
     HIPTRY(hipEventRecord(ev0_, stream_));
+    const double pass_bytes = 32.0 * (double)num_;
+    auto row_pass = [&](size_t segment) {
+        prof_.begin(KC_ROWS, pass_bytes);
+        const hipError_t e = launch_rows(d_re_, d_im_, d_rows_ + row_first_[segment], n_, stream_);
+        prof_.end();
+        last_launches_++;
+        return e;
+    };
+    auto transpose = [&] {
+        prof_.begin(KC_TRANSPOSE, pass_bytes);
+        const hipError_t e = launch_conj_transpose(d_re_, d_im_, n_, stream_);
+        prof_.end();
+        last_launches_++;
+        return e;
+    };
     // Segments of gate primitives between channels: each segment runs its two
     // index passes (the reference's forward and backward pass); a channel then
     // acts once on both indices, in the record for the current orientation.
     int s0 = 0;
+    size_t segment = 0;
     while (s0 < n_ops) {
         int s1 = s0;
         while (s1 < n_ops && prims_[s1].kind != PK_SUP) s1++;
-        if (s1 > s0) {
+        if (s1 > s0 && rows) {
+            // the reference's order: columns, conjugate transpose, columns
+            if (transposed_) HIPTRY(transpose());
+            transposed_ = false;
+            HIPTRY(row_pass(segment));
+            HIPTRY(transpose());
+            HIPTRY(row_pass(segment));
+            segment++;
+            last_sweeps_ += 2u * (uint32_t)(s1 - s0);
+        } else if (s1 > s0) {
             // reference orientation: fast index first; transposed: slow first
             const bool first_slow = transposed_;
             for (int pass = 0; pass < 2; pass++) {
                 const bool slow = pass == 0 ? first_slow : !first_slow;
-                int t = s0;
-                while (t < s1) {
-                    if (per_launch || prims_[t].kind == PK_C2) {
-                        prof_.begin(prim_class(prims_[t]), prim_bytes(prims_[t], n_));
-                        HIPTRY(launch_plain_one(d_re_, d_im_, d_ops_ + t, prims_[t], n_, slow,
-                                                max_blocks_, stream_));
-                        prof_.end();
-                        last_launches_++;
-                        t++;
-                        continue;
-                    }
-                    int end = t;
-                    double bytes = 0;
-                    while (end < s1 && prims_[end].kind != PK_C2)
-                        bytes += prim_bytes(prims_[end++], n_);
-                    hipError_t e = hipErrorCooperativeLaunchTooLarge;
-                    if (coop_ok) {
-                        prof_.begin(KC_PERSISTENT, bytes);
-                        e = launch_plain_persistent(d_re_, d_im_, d_ops_, t, end, n_, slow,
-                                                    persistent_blocks_, stream_);
-                        prof_.end();
-                    }
-                    if (e == hipSuccess) {
-                        last_launches_++;
-                        t = end;
-                        continue;
-                    }
-                    // The cooperative launch was refused (ROCm grants the
-                    // grid barrier's hardware to one process on a device at
-                    // a time) and did not run: the same primitives, one
-                    // launch each, give the same bits.
-                    (void)hipGetLastError();
-                    if (coop_ok) prof_.cancel();
-                    coop_ok = false;
-                    last_fallbacks_++;
-                    for (; t < end; t++) {
-                        prof_.begin(prim_class(prims_[t]), prim_bytes(prims_[t], n_));
-                        HIPTRY(launch_plain_one(d_re_, d_im_, d_ops_ + t, prims_[t], n_, slow,
-                                                max_blocks_, stream_));
-                        prof_.end();
-                        last_launches_++;
-                    }
+                for (int t = s0; t < s1; t++) {
+                    prof_.begin(prim_class(prims_[t]), prim_bytes(prims_[t], n_));
+                    HIPTRY(launch_plain_one(d_re_, d_im_, d_ops_ + t, prims_[t], n_, slow,
+                                            max_blocks_, stream_));
+                    prof_.end();
+                    last_launches_++;
                 }
             }
             last_sweeps_ += 2u * (uint32_t)(s1 - s0);
@@ -381,7 +407,6 @@ int Engine::run_fused()
 {
     last_launches_ = 0;
     last_sweeps_ = 0;
-    last_fallbacks_ = 0;
     if (!prof_.enabled()) {
         // launch-bound at small n: one graph launch instead of one per step
         RunGraph* rg = nullptr;
@@ -444,6 +469,7 @@ int Engine::clear_circuit()
 {
     circuit_.clear();
     prims_.clear();
+    row_first_.clear();
     drop_graph();
     delete plan_;
     plan_ = nullptr;

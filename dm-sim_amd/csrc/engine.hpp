@@ -10,6 +10,7 @@
 #include "lower.hpp"
 #include "prim.hpp"
 #include "prof.hpp"
+#include "rows.hpp"
 
 namespace dmx {
 
@@ -83,9 +84,9 @@ public:
     double last_ms() const { return last_ms_; }
     uint32_t last_launches() const { return last_launches_; }
     uint32_t last_sweeps() const { return last_sweeps_; }
-    // Persistent-loop segments of the last run that ran as one launch per
-    // primitive because the cooperative launch was refused.
-    uint32_t last_fallbacks() const { return last_fallbacks_; }
+    // Cooperative launches of the last run that were refused and ran another
+    // way: none, as no run makes a cooperative launch.
+    uint32_t last_fallbacks() const { return 0; }
     // Prints the reference's per-run report after every run (off by default).
     void set_report(bool on) { report_ = on; }
     // Device memory this simulation holds (rho, second planes, tables).
@@ -95,6 +96,8 @@ public:
 private:
     int run_plain(bool per_launch);
     int run_fused();
+    // The resident-row program of prims_ on the device (built on first use).
+    int ensure_rows();
     void drop_graph();
     int ensure_ops_capacity(size_t count);
     int to_reference_orientation();
@@ -109,6 +112,9 @@ private:
     double* d_diag_ = nullptr;
     PrimOp* d_ops_ = nullptr;
     size_t d_ops_cap_ = 0;
+    RowOp* d_rows_ = nullptr;  // every segment's program (rows.hpp)
+    size_t d_rows_cap_ = 0;
+    std::vector<size_t> row_first_;  // first record of each; empty: not built
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
 
@@ -122,7 +128,6 @@ private:
     int tuned_tile_bits_ = 0;  // width the last upload's timing chose (0: none)
     bool herm_wanted() const;
     bool permuting_pays(const PlanInfo& perm, const PlanInfo& inplace) const;
-    int persistent_blocks_ = 0;
     int max_blocks_ = 8192;  // grid cap for one-primitive launches
 
     std::vector<Gate> circuit_;
@@ -152,7 +157,6 @@ private:
     double last_ms_ = 0.0;
     uint32_t last_launches_ = 0;
     uint32_t last_sweeps_ = 0;
-    uint32_t last_fallbacks_ = 0;
     bool report_ = false;
 };
 

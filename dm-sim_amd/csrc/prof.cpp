@@ -5,7 +5,8 @@ namespace dmx {
 
 const char* const kKernelClassNames[KC_COUNT] = {
     "k_fused4", "k_sweep(dense pair)", "k_sweep(diagonal pair)", "k_sweep(cx)", "k_quad",
-    "k_plain_persistent", "k_fused5", "k_fused4_perm", "k_fused4_herm", "k_relabel"};
+    "k_rows", "k_fused5", "k_fused4_perm", "k_fused4_herm", "k_relabel",
+    "k_conj_transpose"};
 
 LaunchProfiler::~LaunchProfiler()
 {
@@ -43,11 +44,6 @@ void LaunchProfiler::end()
     if (!on_ || recs_.empty()) return;
     recs_.back().b = take();
     if (recs_.back().b) (void)hipEventRecord(recs_.back().b, stream_);
-}
-
-void LaunchProfiler::cancel()
-{
-    if (on_ && !recs_.empty()) recs_.pop_back();
 }
 
 hipError_t LaunchProfiler::collect()

@@ -13,11 +13,12 @@ enum KernelClass : int {
     KC_PAIR_POS1,     // k_sweep, diagonal kinds (only the bit-set entry changes)
     KC_CX,            // k_sweep, controlled swap
     KC_QUAD,          // k_quad, 4x4 primitive
-    KC_PERSISTENT,    // k_plain_persistent, a segment of primitives
+    KC_ROWS,          // k_rows: a segment of primitives on one index, whole rows resident
     KC_FUSED5,        // k_fused5: one dense 5-qubit block, both sides of rho
     KC_FUSED4P,       // k_fused4_perm: a 4-qubit block with a trailing permutation, out of place
     KC_FUSED4H,       // k_fused4_herm: a 4-qubit block on the upper tiles of Hermitian rho, out of place
     KC_RELABEL,       // k_relabel: rho's index bits relabelled, out of place
+    KC_TRANSPOSE,     // k_conj_transpose, in place
     KC_COUNT
 };
 
@@ -37,7 +38,6 @@ public:
     void start(hipStream_t s);  // new run
     void begin(int cls, double bytes);
     void end();
-    void cancel();  // drops the record of the last begin() (its launch did not run)
     hipError_t collect();  // after the stream is synchronised
     const KernelStat& stat(int cls) const { return stats_[cls]; }
 

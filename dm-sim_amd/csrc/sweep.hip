@@ -22,11 +22,11 @@
 // without FMA contraction, so results match the reference CPU path exactly.
 #pragma clang fp contract(off)
 
-#include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
+#include "pair.hpp"
 #include "prim.hpp"
 #include "sweep.hpp"
 
@@ -34,97 +34,10 @@ namespace dmx {
 
 namespace {
 
-constexpr double kS2I = 0.70710678118654752440;  // src/config.hpp:57
-
 __device__ __forceinline__ uint64_t ins0(uint64_t x, int b)
 {
     const uint64_t lo = x & ((1ull << b) - 1);
     return ((x ^ lo) << 1) | lo;
-}
-
-// Output for the pos0 (SEL = 0) or pos1 (SEL = 1) entry of a pair
-// (a0 + i b0, a1 + i b1); expressions as in src/dmsim_amdgpu_omp.hpp:1019-1480.
-template <int K>
-__device__ __forceinline__ void out0(const double* c, double a0, double b0, double a1, double b1,
-                                     double& yr, double& yi)
-{
-    if constexpr (K == PK_C1) {
-        yr = (c[0] * a0) - (c[1] * b0) + (c[2] * a1) - (c[3] * b1);
-        yi = (c[0] * b0) + (c[1] * a0) + (c[2] * b1) + (c[3] * a1);
-    } else if constexpr (K == PK_X) {
-        yr = a1; yi = b1;
-    } else if constexpr (K == PK_Y) {
-        yr = b1; yi = -a1;
-    } else if constexpr (K == PK_H) {
-        yr = kS2I * (a0 + a1); yi = kS2I * (b0 + b1);
-    } else if constexpr (K == PK_SRN) {
-        yr = 0.5 * (a0 + a1); yi = 0.5 * (b0 - b1);
-    } else if constexpr (K == PK_RX) {
-        yr = (c[0] * a0) - (c[1] * b1); yi = (c[0] * b0) + (c[1] * a1);
-    } else if constexpr (K == PK_RY) {
-        yr = (c[0] * a0) + (c[1] * a1); yi = (c[0] * b0) + (c[1] * b1);
-    } else if constexpr (K == PK_W) {
-        yr = kS2I * (a0 + b1); yi = kS2I * (b0 - a1);
-    } else {  // pos1-only kinds keep pos0
-        yr = a0; yi = b0;
-    }
-}
-
-template <int K>
-__device__ __forceinline__ void out1(const double* c, double a0, double b0, double a1, double b1,
-                                     double& yr, double& yi)
-{
-    if constexpr (K == PK_C1) {
-        yr = (c[4] * a0) - (c[5] * b0) + (c[6] * a1) - (c[7] * b1);
-        yi = (c[4] * b0) + (c[5] * a0) + (c[6] * b1) + (c[7] * a1);
-    } else if constexpr (K == PK_X) {
-        yr = a0; yi = b0;
-    } else if constexpr (K == PK_Y) {
-        yr = -b0; yi = a0;
-    } else if constexpr (K == PK_H) {
-        yr = kS2I * (a0 - a1); yi = kS2I * (b0 - b1);
-    } else if constexpr (K == PK_SRN) {
-        yr = 0.5 * (a0 + a1); yi = 0.5 * (-b0 + b1);
-    } else if constexpr (K == PK_RX) {
-        yr = -(c[1] * b0) + (c[0] * a1); yi = (c[1] * a0) + (c[0] * b1);
-    } else if constexpr (K == PK_RY) {
-        yr = (c[2] * a0) + (c[3] * a1); yi = (c[2] * b0) + (c[3] * b1);
-    } else if constexpr (K == PK_W) {
-        yr = kS2I * (b0 + a1); yi = kS2I * (-a0 + b1);
-    } else if constexpr (K == PK_Z) {
-        yr = -a1; yi = -b1;
-    } else if constexpr (K == PK_S) {
-        yr = -b1; yi = a1;
-    } else if constexpr (K == PK_SDG) {
-        yr = b1; yi = -a1;
-    } else if constexpr (K == PK_T) {
-        yr = kS2I * (a1 - b1); yi = kS2I * (a1 + b1);
-    } else if constexpr (K == PK_TDG) {
-        yr = kS2I * (a1 + b1); yi = kS2I * (-a1 + b1);
-    } else if constexpr (K == PK_R) {
-        yr = -(b1 * c[0]); yi = a1 * c[0];
-    } else if constexpr (K == PK_U1) {
-        yr = (c[0] * a1) - (c[1] * b1); yi = (c[0] * b1) + (c[1] * a1);
-    }
-}
-
-// CJ: evaluate on conjugated operands and conjugate the result (slow index).
-template <int K, bool CJ>
-__device__ __forceinline__ void eval0(const double* c, double a0, double b0, double a1, double b1,
-                                      double& yr, double& yi)
-{
-    if constexpr (CJ) { b0 = -b0; b1 = -b1; }
-    out0<K>(c, a0, b0, a1, b1, yr, yi);
-    if constexpr (CJ) yi = -yi;
-}
-
-template <int K, bool CJ>
-__device__ __forceinline__ void eval1(const double* c, double a0, double b0, double a1, double b1,
-                                      double& yr, double& yi)
-{
-    if constexpr (CJ) { b0 = -b0; b1 = -b1; }
-    out1<K>(c, a0, b0, a1, b1, yr, yi);
-    if constexpr (CJ) yi = -yi;
 }
 
 __device__ __forceinline__ double2 ld2(const double* p)
@@ -325,75 +238,9 @@ __device__ void sweep_quad(double* __restrict__ re, double* __restrict__ im,
     }
 }
 
-// Persistent-loop dispatch of one pair primitive (4x4 sweeps are launched
-// separately; see plain_segments()).
-template <bool SLOW>
-__device__ void run_pair(const PrimOp* __restrict__ op, double* re, double* im, int n)
-{
-    const uint64_t N = 1ull << (2 * n);
-    const int shift = SLOW ? n : 0;
-    const int kind = op->kind;
-    const int b = op->q0 + shift;
-    const int cb = op->q1 >= 0 ? op->q1 + shift : -1;
-    const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t gthreads = (uint64_t)gridDim.x * blockDim.x;
-    const Range waves{gtid >> 6, gthreads >> 6, (int)(threadIdx.x & 63)};
-    const Range threads{gtid, gthreads, 0};
-    double c[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) c[i] = op->c[i];
-#define DMX_PAIR_CASE(KK)                                                             \
-    case KK:                                                                          \
-        if (N < 256)                                                                  \
-            sweep_tiny<KK, SLOW>(re, im, c, b, cb, N, threads);                       \
-        else if (b >= 7)                                                              \
-            sweep_wide<KK, SLOW>(re, im, c, b, cb < 0 ? -1 : (cb < b ? cb : cb - 1), N, \
-                                 waves);                                              \
-        else                                                                          \
-            sweep_narrow<KK, SLOW>(re, im, c, b, cb, N, waves);                       \
-        break;
-    switch (kind) {
-        DMX_PAIR_CASE(PK_C1)
-        DMX_PAIR_CASE(PK_X)
-        DMX_PAIR_CASE(PK_Y)
-        DMX_PAIR_CASE(PK_H)
-        DMX_PAIR_CASE(PK_SRN)
-        DMX_PAIR_CASE(PK_RX)
-        DMX_PAIR_CASE(PK_RY)
-        DMX_PAIR_CASE(PK_W)
-        DMX_PAIR_CASE(PK_Z)
-        DMX_PAIR_CASE(PK_S)
-        DMX_PAIR_CASE(PK_SDG)
-        DMX_PAIR_CASE(PK_T)
-        DMX_PAIR_CASE(PK_TDG)
-        DMX_PAIR_CASE(PK_R)
-        DMX_PAIR_CASE(PK_U1)
-    default:
-        break;
-    }
-#undef DMX_PAIR_CASE
-}
-
 enum Path { P_TINY = 0, P_NARROW = 1, P_WIDE = 2 };
 
 }  // namespace
-
-// Persistent gate loop: primitives [first, last) of one pass in a single
-// cooperative launch with a grid barrier after every primitive (the
-// reference's BSP structure, src/dmsim_amdgpu_omp.hpp:831-837, :1004-1016).
-__global__ void __launch_bounds__(256) k_plain_persistent(double* re, double* im,
-                                                          const PrimOp* __restrict__ ops,
-                                                          int first, int last, int n, int slow)
-{
-    cooperative_groups::grid_group grid = cooperative_groups::this_grid();
-    for (int t = first; t < last; t++) {
-        if (slow)
-            run_pair<true>(ops + t, re, im, n);
-        else
-            run_pair<false>(ops + t, re, im, n);
-        if (t + 1 < last) grid.sync();
-    }
-}
 
 // One pair primitive per launch, specialised by kind, index side and access
 // path (each instance keeps its own small register budget).
@@ -542,45 +389,6 @@ SweepFn sweep_fn(int kind, int path)
 }
 
 }  // namespace
-
-hipError_t plain_persistent_grid(int n, int* blocks)
-{
-    int per_cu = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, reinterpret_cast<const void*>(k_plain_persistent), 256, 0);
-    if (e != hipSuccess) return e;
-    int dev = 0;
-    e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    int cus = 0;
-    e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return e;
-    // The grid barrier after every primitive costs more the more blocks take
-    // part: N / 8192 blocks, at least 16, at most 256 (n <= 12) or 512, one wave
-    // per 256 entries at most, measured fastest from n = 8 to n = 14 (16.2 ms
-    // for 1000 gates at n = 8, 31 ms for 600 at n = 10, 52 ms for 200 at n = 12,
-    // 342 ms for 120 at n = 14, against 23, 170, 100 and 365 ms with every
-    // co-resident block).
-    const uint64_t N = 1ull << (2 * n);
-    uint64_t g = N / 8192;
-    if (g < 16) g = 16;
-    if (g > (n <= 12 ? 256u : 512u)) g = n <= 12 ? 256 : 512;
-    const uint64_t most = (N / 1024) > 0 ? (N / 1024) : 1;  // one wave per 256 entries
-    if (g > most) g = most;
-    if (g > (uint64_t)per_cu * (uint64_t)cus) g = (uint64_t)per_cu * (uint64_t)cus;
-    if (g < 1) g = 1;
-    *blocks = (int)g;
-    return hipSuccess;
-}
-
-hipError_t launch_plain_persistent(double* re, double* im, const PrimOp* d_ops, int first,
-                                   int last, int n, bool slow, int blocks, hipStream_t stream)
-{
-    int sl = slow ? 1 : 0;
-    void* args[] = {&re, &im, const_cast<PrimOp**>(&d_ops), &first, &last, &n, &sl};
-    return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k_plain_persistent),
-                                      dim3(blocks), dim3(256), args, 0, stream);
-}
 
 hipError_t launch_plain_one(double* re, double* im, const PrimOp* d_op, const PrimOp& host_op,
                             int n, bool slow, int max_blocks, hipStream_t stream)

@@ -7,16 +7,6 @@
 
 namespace dmx {
 
-// Blocks of 256 threads for the persistent loop: 4^n / 8192 clamped to
-// 16..256 (n <= 12) or 16..512, at most one wave per 256 entries of a plane
-// and at most the co-resident maximum on this device.
-hipError_t plain_persistent_grid(int n, int* blocks);
-
-// Pair primitives [first, last) of one pass (slow: row index) in one
-// cooperative launch.  4x4 primitives are not accepted here.
-hipError_t launch_plain_persistent(double* re, double* im, const PrimOp* d_ops, int first,
-                                   int last, int n, bool slow, int blocks, hipStream_t stream);
-
 // One primitive sweep; host_op is the host copy of *d_op (selects the kernel).
 hipError_t launch_plain_one(double* re, double* im, const PrimOp* d_op, const PrimOp& host_op,
                             int n, bool slow, int max_blocks, hipStream_t stream);

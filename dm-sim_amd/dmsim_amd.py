@@ -343,8 +343,7 @@ class Sim:
         _check(load().dmx_last_run_stats(self._h, C.byref(ms), C.byref(la), C.byref(sw)))
         fb = C.c_uint32()
         _check(load().dmx_last_run_fallbacks(self._h, C.byref(fb)))
-        # fallbacks: persistent-loop segments run one launch per primitive
-        # because the cooperative launch was refused
+        # fallbacks: refused cooperative launches (none are made)
         return {"ms": ms.value, "launches": la.value, "sweeps": sw.value,
                 "fallbacks": fb.value}
 

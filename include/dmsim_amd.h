@@ -43,8 +43,8 @@ enum dmx_op {
 };
 
 /* Execution methods (dmx_set_method). */
-#define DMX_METHOD_PLAIN 0        /* persistent cooperative gate loop, 2 sweeps per primitive */
-#define DMX_METHOD_PLAIN_LAUNCH 1 /* same sweeps, one launch per primitive                    */
+#define DMX_METHOD_PLAIN 0        /* gate by gate, whole rows of rho on chip (n <= 14)           */
+#define DMX_METHOD_PLAIN_LAUNCH 1 /* gate by gate, 2 sweeps and launches per primitive           */
 #define DMX_METHOD_FUSED 2        /* gates fused into dense 4- and 5-qubit blocks, one sweep each */
 
 typedef struct dmx_sim dmx_sim;
@@ -194,12 +194,12 @@ int dmx_last_run_stats(const dmx_sim* sim, double* ms, uint32_t* launches, uint3
  * C ABI's default) is silent.  The C++ and Python faces turn it on. */
 int dmx_set_report(dmx_sim* sim, int on);
 
-/* Extension: how many persistent-loop segments of the last DMX_METHOD_PLAIN
- * run fell back to one launch per primitive (bit-identical results) because
- * the device refused the cooperative launch, as ROCm does while another
- * process holds the device's grid-barrier resource.  The reference's
- * hipLaunchCooperativeKernel call (src/dmsim_amdgpu_omp.hpp:420-433) exits
- * the process in that case. */
+/* Extension: how many segments of the last run fell back to one launch per
+ * primitive because the device refused a cooperative launch, as ROCm does
+ * while another process holds the device's grid-barrier resource.  No method
+ * makes cooperative launches (rows of rho need no grid barrier), so 0.  The
+ * reference's hipLaunchCooperativeKernel call
+ * (src/dmsim_amdgpu_omp.hpp:420-433) exits the process in that case. */
 int dmx_last_run_fallbacks(const dmx_sim* sim, uint32_t* segments);
 
 /* Extension: time every launch of subsequent runs with a pair of HIP events on
