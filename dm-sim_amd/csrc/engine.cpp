@@ -160,8 +160,9 @@ int Engine::upload()
     if (method_ == DMX_METHOD_FUSED) {
         // no plan (SRN in the circuit, or n < 4): the run uses the plain sweeps
         const bool herm = herm_wanted();
+        const bool fold = n_ >= kFoldChannelQubits;
         int rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_,
-                                  fusion_permute_, &plan_, &plan_info_, herm);
+                                  fusion_permute_, &plan_, &plan_info_, herm, fold);
         if (rc) return rc;
         if (plan_ && plan_info_.perm_blocks > 0 && n_ < kPermuteSureQubits && fusion_herm_ != 2) {
             // a short sweep is latency-bound and a permuting one pays its index
@@ -169,7 +170,7 @@ int Engine::upload()
             FusedPlan* inplace = nullptr;
             PlanInfo ii;
             rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_, false,
-                                  &inplace, &ii);
+                                  &inplace, &ii, false, fold);
             if (rc) return rc;
             if (inplace && !permuting_pays(plan_info_, ii)) {
                 drop_graph();
@@ -197,7 +198,7 @@ int Engine::upload()
                 delete plan_;
                 plan_ = nullptr;
                 rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_, false,
-                                      &plan_, &plan_info_);
+                                      &plan_, &plan_info_, false, fold);
                 if (rc) return rc;
             }
         }
@@ -407,6 +408,10 @@ int Engine::run_fused()
 {
     last_launches_ = 0;
     last_sweeps_ = 0;
+    if (plan_->staged()) {  // a block's channels have one record, for the stored orientation
+        const int rc = to_reference_orientation();
+        if (rc) return rc;
+    }
     if (!prof_.enabled()) {
         // launch-bound at small n: one graph launch instead of one per step
         RunGraph* rg = nullptr;

@@ -59,6 +59,9 @@ struct FusedPlan {
     virtual ~FusedPlan() = default;
     virtual void describe(std::vector<PlanStepView>& out) const = 0;
     virtual int upload(hipStream_t stream) = 0;
+    // Whether blocks hold channels (FusedStage): execute then takes rho in its
+    // stored orientation only (transposed = false).
+    virtual bool staged() const = 0;
     // Whether execute needs a second pair of planes (blocks with a trailing
     // permutation run out of place).
     virtual bool needs_alt() const = 0;
@@ -94,6 +97,7 @@ struct BlockPlan {
     std::vector<int> dense;
     std::vector<FusedBlock5> blocks5;
     std::vector<std::vector<int>> members5;
+    std::vector<FusedStage> stages;  // of the blocks with channels
     std::vector<std::pair<int, int>> order;
 };
 
@@ -114,9 +118,12 @@ struct BlockPlan {
 // cheaper of its fused sweep and its gates unfused); without a model the one
 // with fewer sweeps of the first two.  *grouping (may be null) = the choice:
 // 0..5 in that order.
+// fold: a channel is a member of a block like a one-qubit gate, and a block
+// with channels runs as stages (unless a gate is wider than four qubits:
+// channels then stand between blocks, as without fold).
 int plan_blocks(const std::vector<Gate>& circuit, int n, int max_k, BlockPlan& out, bool& fusable,
                 bool allow_perm = false, bool herm = false, CostModel* model = nullptr,
-                uint32_t* grouping = nullptr);
+                uint32_t* grouping = nullptr, bool fold = false);
 
 // Relative extra cost of a sweep with a trailing permutation on n qubits:
 // about 2.5 us of index-map set-up against the sweep's own time (32 * 4^n bytes
@@ -155,7 +162,14 @@ inline bool permuting_pays(int n, double sweeps, double permuting, double sweeps
 // circuit's bit order (k_relabel) before any other step and at the end.
 int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model,
                      int tile_bits, bool allow_perm, FusedPlan** out, PlanInfo* info,
-                     bool herm = false);
+                     bool herm = false, bool fold = false);
+
+// From this many qubits the engine folds channels into blocks.  A noisy
+// 318-member circuit at 8 qubits takes 9 sweeps instead of 138 and 180 channel
+// sweeps (1.32 -> 0.22 ms a run with its downloads), one of 164 members at 12
+// qubits 12 instead of 182 launches (16.1 -> 1.95 ms).  Below, a plan's launches
+// stay one per block and channel, which callers at those sizes count on.
+constexpr int kFoldChannelQubits = 7;
 
 // Smallest n for Hermitian plans, and the smallest where the engine uses
 // them by default.

@@ -91,6 +91,99 @@ __device__ __forceinline__ uint64_t deposit(uint64_t v, uint64_t mask)
     return out;
 }
 
+// The stages of a block with channels, on the workgroup's super-tile in LDS.
+// Each wave takes its own tiles (tb = wave, wave + 4, ...; those with
+// on(tb)) through all stages, so there is no barrier between stages; a
+// stage's matrix is loaded once for the wave's tiles.  col(tb, b): LDS column of
+// local column b of tile tb; at(a, x): LDS place of row a, column x.
+// A superoperator stage is Y = S X with X's rows the 16 (row, column) values of
+// bits u, v and X's columns the 16 of the other two: 12 MFMAs (one complex
+// product) against the 24 of a unitary stage, and a lane reads and writes the
+// same four places.  Bound like the sweep around it by memory up to about four
+// stages a block (4 stages of 12 MFMAs take as long as a Hermitian sweep's
+// traffic at 60 TFLOP/s), by the FP64 MFMA rate above: at n = 14, 38 noisy
+// sweeps take 1.51 ms each where 32 unitary ones take 0.98.
+template <int NTILES, class On, class Col, class At>
+__device__ __forceinline__ void run_stages(const FusedStage* __restrict__ stages, uint32_t count,
+                                           int wave, int lane, const On& on, const Col& col,
+                                           const At& at, double* __restrict__ s_re,
+                                           double* __restrict__ s_im)
+{
+    const int j = lane & 15;
+    const int kk = lane >> 4;
+    for (uint32_t s = 0; s < count; s++) {
+        const FusedStage& g = stages[s];
+        double ur[4], ui[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            ur[c] = g.re[j * 16 + 4 * c + kk];
+            ui[c] = g.im[j * 16 + 4 * c + kk];
+        }
+        // the wave's earlier writes, from other lanes, come before these reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (g.whole) {
+            for (int tb = wave; tb < NTILES; tb += 4) {
+                if (!on(tb)) continue;
+                d4 p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int x = at(j, col(tb, 4 * c + kk));
+                    const double tr = s_re[x], ti = s_im[x];
+                    p1 = mfma(tr, ur[c], p1);
+                    p2 = mfma(ti, ui[c], p2);
+                    p3 = mfma(tr + ti, ur[c] + ui[c], p3);
+                }
+                const d4 xr = p1 - p2;
+                const d4 xi = p3 - p1 - p2;
+                d4 q1 = {0, 0, 0, 0}, q2 = {0, 0, 0, 0}, q3 = {0, 0, 0, 0};
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    q1 = mfma(ur[c], xr[c], q1);
+                    q2 = mfma(-ui[c], xi[c], q2);
+                    q3 = mfma(ur[c] - ui[c], xr[c] + xi[c], q3);
+                }
+                const d4 yr = q1 - q2;
+                const d4 yi = q3 - q1 - q2;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int x = at(4 * r + kk, col(tb, j));
+                    s_re[x] = yr[r];
+                    s_im[x] = yi[r];
+                }
+            }
+            continue;
+        }
+        const int spec_r = ((j >> 2) & 1) << g.x | (j >> 3) << g.y;
+        const int b = (kk & 1) << g.u | (kk >> 1) << g.v | (j & 1) << g.x | ((j >> 1) & 1) << g.y;
+        int row[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) row[c] = spec_r | (c & 1) << g.u | (c >> 1) << g.v;
+        for (int tb = wave; tb < NTILES; tb += 4) {
+            if (!on(tb)) continue;
+            const int x0 = col(tb, b);
+            d4 p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int x = at(row[c], x0);
+                const double tr = s_re[x], ti = s_im[x];
+                p1 = mfma(ur[c], tr, p1);
+                p2 = mfma(ui[c], ti, p2);
+                p3 = mfma(ur[c] + ui[c], tr + ti, p3);
+            }
+            const d4 yr = p1 - p2;
+            const d4 yi = p3 - p1 - p2;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int x = at(row[r], x0);
+                s_re[x] = yr[r];
+                s_im[x] = yi[r];
+            }
+        }
+    }
+}
+
 }  // namespace
 
 // Super-tiles st_first, st_first + st_stride, ... of one block sweep; s_re and
@@ -99,11 +192,13 @@ __device__ __forceinline__ uint64_t deposit(uint64_t v, uint64_t mask)
 // PERM: the block has a trailing permutation pi; super-tiles are read from
 // (re, im) and written, entry (i, j) to (pi(i), pi(j)), into (re_out, im_out).
 // Otherwise re_out/im_out are re/im (in place).
-template <int M, bool PERM = false, bool PIPE = false>
+// STAGED: the block's tiles pass through its stages (run_stages).
+template <int M, bool PERM = false, bool PIPE = false, bool STAGED = false>
 __device__ __forceinline__ void fused_sweep(double* re, double* im, double* re_out,
                                             double* im_out, const FusedBlock* __restrict__ blk,
                                             int n, uint64_t st_first, uint64_t st_stride,
-                                            double* __restrict__ s_re, double* __restrict__ s_im)
+                                            double* __restrict__ s_re, double* __restrict__ s_im,
+                                            const FusedStage* __restrict__ stages = nullptr)
 {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -227,7 +322,12 @@ __device__ __forceinline__ void fused_sweep(double* re, double* im, double* re_o
         __syncthreads();
         if (PIPE && active && st + st_stride < n_st) load(base_of(st + st_stride));
 
-        for (int tb = wave; tb < ntiles; tb += 4) {
+        if constexpr (STAGED)
+            run_stages<ntiles>(
+                stages + blk->stage0, blk->stages, wave, lane, [](int) { return true; },
+                [&](int tb, int b) { return (int)(deposit(tb, pos_f) | deposit(b, pos_q)); },
+                [](int a, int x) { return lds_at(a, x); }, s_re, s_im);
+        for (int tb = wave; tb < ntiles && !STAGED; tb += 4) {
             const uint32_t base = (uint32_t)deposit((uint64_t)tb, pos_f);
             double tr[4], ti[4], ts[4];
 #pragma unroll
@@ -308,6 +408,21 @@ __global__ void __launch_bounds__(256, 2) k_fused4(double* __restrict__ re, doub
     fused_sweep<M, false, PIPE>(re, im, re, im, blk, n, blockIdx.x, gridDim.x, s_re, s_im);
 }
 
+// A block with noise channels among its gates (its stages), in place or, with a
+// trailing permutation, out of place.
+template <int M, bool PERM>
+__global__ void __launch_bounds__(256, 2) k_fused4_staged(double* re, double* im, double* re_out,
+                                                           double* im_out,
+                                                           const FusedBlock* __restrict__ blk,
+                                                           const FusedStage* __restrict__ stages,
+                                                           int n)
+{
+    __shared__ double s_re[16 * kPitch];
+    __shared__ double s_im[16 * kPitch];
+    fused_sweep<M, PERM, false, true>(re, im, re_out, im_out, blk, n, blockIdx.x, gridDim.x, s_re,
+                                      s_im, stages);
+}
+
 template <int M, bool PIPE>
 __global__ void __launch_bounds__(256, 2) k_fused4_perm(const double* __restrict__ re,
                                                          const double* __restrict__ im,
@@ -354,14 +469,16 @@ __global__ void __launch_bounds__(256, 2) k_fused4_batch(const BatchEntry* __res
 // next(k, w) sets w to its k-th item and returns false once they are used up
 // (then for every later k as well).  NT: nontemporal loads and stores (rho
 // streamed from HBM); without, cached ones (rho in the Infinity Cache).
-template <bool NT, bool PIPE, class Next>
+// STAGED: the tiles pass through the block's stages (run_stages).
+template <bool NT, bool PIPE, bool STAGED, class Next>
 __device__ __forceinline__ void herm_sweep(const double* __restrict__ re,
                                            const double* __restrict__ im,
                                            double* __restrict__ re_out,
                                            double* __restrict__ im_out,
                                            const FusedBlock* __restrict__ blk, const HermGeom& g,
                                            Next next, double* __restrict__ s_re,
-                                           double* __restrict__ s_im)
+                                           double* __restrict__ s_im,
+                                           const FusedStage* __restrict__ stages = nullptr)
 {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -420,7 +537,13 @@ __device__ __forceinline__ void herm_sweep(const double* __restrict__ re,
         have = next(k + 1, w);
         if (PIPE && have) load();
 
-        for (int tb = wave; tb < 16; tb += 4) {
+        if constexpr (STAGED)
+            run_stages<16>(
+                stages + blk->stage0, blk->stages, wave, lane,
+                [&](int tb) { return herm_tile_on(cur, tb); },
+                [&](int tb, int b) { return (int)(deposit(tb, g.pos_f) | (uint32_t)th.dq(b)); },
+                [](int a, int x) { return herm_lds(a, x); }, s_re, s_im);
+        for (int tb = wave; tb < 16 && !STAGED; tb += 4) {
             if (!herm_tile_on(cur, tb)) continue;
             const uint32_t base = (uint32_t)deposit((uint64_t)tb, g.pos_f);
             double tr[4], ti[4], ts[4];
@@ -491,11 +614,28 @@ __global__ void __launch_bounds__(256, 2) k_fused4_herm(const double* __restrict
     __shared__ double s_im[16 * kHermPitch];
     HermGeom g;
     g.init(*blk, n);
-    herm_sweep<true, true>(re, im, re_out, im_out, blk, g,
+    herm_sweep<true, true, false>(re, im, re_out, im_out, blk, g,
                      [&](uint64_t k, uint64_t& w) {
                          return herm_slot(g, blockIdx.x, gridDim.x, k, w);
                      },
                      s_re, s_im);
+}
+
+// The same for a block with noise channels among its gates.
+__global__ void __launch_bounds__(256, 2) k_fused4_herm_staged(
+    const double* __restrict__ re, const double* __restrict__ im, double* __restrict__ re_out,
+    double* __restrict__ im_out, const FusedBlock* __restrict__ blk,
+    const FusedStage* __restrict__ stages, int n)
+{
+    __shared__ double s_re[16 * kHermPitch];
+    __shared__ double s_im[16 * kHermPitch];
+    HermGeom g;
+    g.init(*blk, n);
+    herm_sweep<true, true, true>(re, im, re_out, im_out, blk, g,
+                                 [&](uint64_t k, uint64_t& w) {
+                                     return herm_slot(g, blockIdx.x, gridDim.x, k, w);
+                                 },
+                                 s_re, s_im, stages);
 }
 
 // Batched form: blockIdx.y selects one circuit's (rho, block) pair, all of
@@ -511,7 +651,7 @@ __global__ void __launch_bounds__(256, 2) k_fused4_herm_batch(const BatchEntry* 
     HermGeom g;
     g.init(*e.blk, n);
     const uint64_t items = g.items();
-    herm_sweep<NT, PIPE>(e.re, e.im, e.re_out, e.im_out, e.blk, g,
+    herm_sweep<NT, PIPE, false>(e.re, e.im, e.re_out, e.im_out, e.blk, g,
                       [&](uint64_t k, uint64_t& w) {
                           w = blockIdx.x + k * gridDim.x;
                           return w < items;
@@ -603,12 +743,39 @@ constexpr int kBatchHermStreamQubits = 10;
 
 }  // namespace
 
+namespace {
+
+template <bool PERM>
+hipError_t launch_staged(double* re, double* im, double* re_out, double* im_out,
+                         const FusedBlock* d_blk, const FusedStage* d_stages, int n, int m,
+                         unsigned blocks, hipStream_t stream)
+{
+#define DMX_STAGED_CASE(MM)                                                                     \
+    case MM:                                                                                   \
+        k_fused4_staged<MM, PERM><<<blocks, 256, 0, stream>>>(re, im, re_out, im_out, d_blk,    \
+                                                              d_stages, n);                    \
+        break;
+    switch (m) {
+        DMX_STAGED_CASE(4)
+        DMX_STAGED_CASE(5)
+        DMX_STAGED_CASE(6)
+        DMX_STAGED_CASE(7)
+        DMX_STAGED_CASE(8)
+    }
+#undef DMX_STAGED_CASE
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_fused4(double* re, double* im, const FusedBlock* d_blk, int n, int m,
-                         int max_blocks, hipStream_t stream)
+                         int max_blocks, hipStream_t stream, const FusedStage* d_stages)
 {
     if (n < 4 || m < 4 || m > 8 || m > n) return hipErrorInvalidValue;
     const uint64_t n_st = supertiles(n, m);
     const unsigned blocks = (unsigned)(n_st < (uint64_t)max_blocks ? n_st : (uint64_t)max_blocks);
+    if (d_stages)
+        return launch_staged<false>(re, im, re, im, d_blk, d_stages, n, m, blocks, stream);
     const bool pipe = n >= kPipeQubits;
     switch (m * 2 + (pipe ? 1 : 0)) {
     case 8: k_fused4<4, false><<<blocks, 256, 0, stream>>>(re, im, d_blk, n); break;
@@ -627,12 +794,15 @@ hipError_t launch_fused4(double* re, double* im, const FusedBlock* d_blk, int n,
 
 hipError_t launch_fused4_perm(const double* re, const double* im, double* re_out, double* im_out,
                               const FusedBlock* d_blk, int n, int m, int max_blocks,
-                              hipStream_t stream)
+                              hipStream_t stream, const FusedStage* d_stages)
 {
     if (n < 4 || n > 16 || m < 4 || m > 8 || m > n || re == re_out || im == im_out)
         return hipErrorInvalidValue;
     const uint64_t n_st = supertiles(n, m);
     const unsigned blocks = (unsigned)(n_st < (uint64_t)max_blocks ? n_st : (uint64_t)max_blocks);
+    if (d_stages)
+        return launch_staged<true>(const_cast<double*>(re), const_cast<double*>(im), re_out, im_out,
+                                   d_blk, d_stages, n, m, blocks, stream);
     const bool pipe = n >= kPipeQubits;
 #define DMX_PERM_CASE(MM)                                                                  \
     case MM:                                                                              \
@@ -659,14 +829,18 @@ hipError_t launch_fused4_perm(const double* re, const double* im, double* re_out
 
 hipError_t launch_fused4_herm(const double* re, const double* im, double* re_out,
                               double* im_out, const FusedBlock* d_blk, int n, int max_blocks,
-                              hipStream_t stream)
+                              hipStream_t stream, const FusedStage* d_stages)
 {
     if (n < 8 || n > 16 || re == re_out || im == im_out) return hipErrorInvalidValue;
     const uint64_t H = 1ull << (n - 8);
     const uint64_t items = 16 * (H * (H + 1) / 2);
     // a multiple of 128 workgroups (herm_slot): 16 per XCD group
     uint64_t blocks = ((items < (uint64_t)max_blocks ? items : (uint64_t)max_blocks) + 127) / 128 * 128;
-    k_fused4_herm<<<(unsigned)blocks, 256, 0, stream>>>(re, im, re_out, im_out, d_blk, n);
+    if (d_stages)
+        k_fused4_herm_staged<<<(unsigned)blocks, 256, 0, stream>>>(re, im, re_out, im_out, d_blk,
+                                                                   d_stages, n);
+    else
+        k_fused4_herm<<<(unsigned)blocks, 256, 0, stream>>>(re, im, re_out, im_out, d_blk, n);
     return hipGetLastError();
 }
 

@@ -24,7 +24,24 @@ struct FusedBlock {
     // block's output order (its sweep reads only the tiles on and above its
     // diagonal, so only those entries are written), 0 = write every entry.
     uint32_t next_q;
+    // Noise channels inside the block: its tiles pass through records
+    // [stage0, stage0 + stages) instead of the matrix above; 0 = the matrix.
+    uint32_t stages;
+    uint32_t stage0;
     uint32_t pad;
+};
+
+// One stage of a block with noise channels.  A superoperator of two of the
+// block's local bits u, v (gates and channels on them composed): the 16 x 16
+// matrix acts on the entries of a tile whose row and column differ in those
+// bits only, index 4 * (row bits v, u) + (column bits v, u).  Or a unitary of
+// the whole block, as FusedBlock's.
+struct FusedStage {
+    uint32_t whole;       // 1: a unitary of the block
+    uint32_t u, v, x, y;  // superoperator: its local bits, then the two others
+    uint32_t pad[3];
+    double re[256];
+    double im[256];
 };
 
 // One circuit's rho and the block to apply to it (batched launches).
@@ -71,16 +88,17 @@ hipError_t launch_fused5(double* re, double* im, const FusedBlock5* d_blk, int n
                          int max_blocks, hipStream_t stream);
 
 // rho <- U rho U^dagger for one block (n >= 4), staged in super-tiles of
-// 16 rows x 2^m columns.
+// 16 rows x 2^m columns.  d_stages: the plan's stage records, for a block with
+// channels (its stages > 0) -- here and below; nullptr for one without.
 hipError_t launch_fused4(double* re, double* im, const FusedBlock* d_blk, int n, int m,
-                         int max_blocks, hipStream_t stream);
+                         int max_blocks, hipStream_t stream, const FusedStage* d_stages = nullptr);
 
 // The same for a block with a trailing permutation (perm_on; n <= 16): reads
 // rho from (re, im), writes the permuted result to (re_out, im_out), which
 // must not overlap the input.
 hipError_t launch_fused4_perm(const double* re, const double* im, double* re_out, double* im_out,
                               const FusedBlock* d_blk, int n, int m, int max_blocks,
-                              hipStream_t stream);
+                              hipStream_t stream, const FusedStage* d_stages = nullptr);
 
 // Hermitian form of the block sweep for n = 8..16 (rho Hermitian): reads
 // the tiles on and above the diagonal of (re, im) and writes every entry of
@@ -89,7 +107,7 @@ hipError_t launch_fused4_perm(const double* re, const double* im, double* re_out
 // qmask bits onto bits 0..3 (not checked here).  No overlap of input and output.
 hipError_t launch_fused4_herm(const double* re, const double* im, double* re_out,
                               double* im_out, const FusedBlock* d_blk, int n, int max_blocks,
-                              hipStream_t stream);
+                              hipStream_t stream, const FusedStage* d_stages = nullptr);
 
 // rho's index bits relabelled by a permutation p (perm_L[q] = 1 << p(q)),
 // out of place, n = 8..16.
