@@ -834,8 +834,17 @@ hipError_t launch_fused4_herm(const double* re, const double* im, double* re_out
     if (n < 8 || n > 16 || re == re_out || im == im_out) return hipErrorInvalidValue;
     const uint64_t H = 1ull << (n - 8);
     const uint64_t items = 16 * (H * (H + 1) / 2);
-    // a multiple of 128 workgroups (herm_slot): 16 per XCD group
-    uint64_t blocks = ((items < (uint64_t)max_blocks ? items : (uint64_t)max_blocks) + 127) / 128 * 128;
+    // A multiple of 128 workgroups (herm_slot): 16 per XCD group.  Two per CU run
+    // at a time and each begins with a few us of index-map set-up, so no more
+    // than that while a workgroup has a dozen items or so at most (us a sweep,
+    // 512 against 4096 workgroups: 12 qubits, 2176 items, 82 against 112; 13
+    // qubits, 8448, 265 against 308); at 14 qubits (33280 items) twice as many,
+    // which even out the last wave (980 against 1000 with 512, 1006 with 4096);
+    // above, the set-up is lost in the sweep and the launch deals best
+    // (15 qubits: a run of 76 steps 330 ms with 4096 against 342 with 1024).
+    const uint64_t fit = items < 16384 ? 512 : items < 65536 ? 1024 : ~0ull;
+    const uint64_t cap = fit < (uint64_t)max_blocks ? fit : (uint64_t)max_blocks;
+    const uint64_t blocks = ((items < cap ? items : cap) + 127) / 128 * 128;
     if (d_stages)
         k_fused4_herm_staged<<<(unsigned)blocks, 256, 0, stream>>>(re, im, re_out, im_out, d_blk,
                                                                    d_stages, n);
