@@ -234,7 +234,8 @@ int Batch::upload()
             // method, blocks of up to four qubits, Hermitian sweeps)
             FusedPlan* p = nullptr;
             PlanInfo pi;
-            int rc = build_fused_plan(c.orig, c.n, 4, model_, 0, true, &p, &pi, true);
+            int rc = build_fused_plan(c.orig, c.n, 4, model_, 0, true, &p, &pi, true, true,
+                                      group_wanted(c.orig, c.n));
             if (rc) return rc;
             if (!p) {
                 set_error("batched circuits must be fusable (no SRN)");
@@ -251,6 +252,7 @@ int Batch::upload()
             bool alt = false;
             for (const PlanStepView& v : steps)
                 if (v.kind == PlanStepView::HERM || v.kind == PlanStepView::RELABEL ||
+                    v.kind == PlanStepView::GROUP ||
                     (v.kind == PlanStepView::FUSED4 && v.block->perm_on))
                     alt = !alt;
             c.final_alt = alt;

@@ -162,7 +162,8 @@ int Engine::upload()
         const bool herm = herm_wanted();
         const bool fold = n_ >= kFoldChannelQubits;
         int rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_,
-                                  fusion_permute_, &plan_, &plan_info_, herm, fold);
+                                  fusion_permute_, &plan_, &plan_info_, herm, fold,
+                                  group_wanted(circuit_, n_));
         if (rc) return rc;
         if (plan_ && plan_info_.perm_blocks > 0 && n_ < kPermuteSureQubits && fusion_herm_ != 2) {
             // a short sweep is latency-bound and a permuting one pays its index

@@ -32,6 +32,7 @@
 #include "dmsim_amd.h"
 #include "engine.hpp"
 #include "fused.hpp"
+#include "group.hpp"
 #include "mlp.hpp"
 #include "sweep.hpp"
 
@@ -57,19 +58,21 @@ inline cd mul_add(cd a, cd b, cd c)
 // Hermitian plans add two out-of-place steps: a four-qubit block through
 // k_fused4_herm (its record rewritten for the bit order rho has then), and a
 // relabelling of rho's index bits (k_relabel) back to the circuit's order
-// before any other step and at the end of the run.
+// before any other step and at the end of the run.  Group plans run nothing but
+// group sweeps (k_group, out of place) and that relabelling.
 enum StepType {
     ST_FUSED4 = 0,
     ST_PLAIN = 1,
     ST_FUSED5 = 2,
     ST_CHANNEL = 3,
     ST_HERM = 4,
-    ST_RELABEL = 5
+    ST_RELABEL = 5,
+    ST_GROUP = 6
 };
 
 struct Step {
     int type;
-    int index;  // block index (blocks or blocks5), or first primitive of the segment
+    int index;  // block index (blocks, blocks5 or groups), or first primitive of the segment
     int count;  // primitives in the segment
 };
 
@@ -78,11 +81,18 @@ struct Plan : FusedPlan {
     std::vector<FusedBlock> blocks;
     std::vector<FusedBlock5> blocks5;
     std::vector<FusedStage> stages;  // of the blocks with channels
+    std::vector<GroupBlock> groups;
+    std::vector<GroupStage> gstages;
+    std::vector<double> gmats;
+    bool channels_inside = false;  // a block or group holds channels
     std::vector<PrimOp> prims;
     std::vector<Step> steps;
     FusedBlock* d_blocks = nullptr;
     FusedBlock5* d_blocks5 = nullptr;
     FusedStage* d_stages = nullptr;
+    GroupBlock* d_groups = nullptr;
+    GroupStage* d_gstages = nullptr;
+    double* d_gmats = nullptr;
     PrimOp* d_prims = nullptr;
     int max_blocks = kFusedGridCap;
 
@@ -91,6 +101,9 @@ struct Plan : FusedPlan {
         if (d_blocks) (void)hipFree(d_blocks);
         if (d_blocks5) (void)hipFree(d_blocks5);
         if (d_stages) (void)hipFree(d_stages);
+        if (d_groups) (void)hipFree(d_groups);
+        if (d_gstages) (void)hipFree(d_gstages);
+        if (d_gmats) (void)hipFree(d_gmats);
         if (d_prims) (void)hipFree(d_prims);
     }
 
@@ -117,13 +130,21 @@ struct Plan : FusedPlan {
         return blocks[block].stages > 0 ? d_stages : nullptr;
     }
 
-    bool staged() const override { return !stages.empty(); }
+    bool staged() const override { return channels_inside; }
+
+    bool five(int group) const
+    {
+        const GroupBlock& b = groups[group];
+        for (uint32_t i = b.stage0; i < b.stage0 + b.stages; i++)
+            if (gstages[i].kind == GS_UNITARY5) return true;
+        return false;
+    }
 
     bool needs_alt() const override
     {
         for (const Step& st : steps)
             if ((st.type == ST_FUSED4 && blocks[st.index].perm_on) || st.type == ST_HERM ||
-                st.type == ST_RELABEL)
+                st.type == ST_RELABEL || st.type == ST_GROUP)
                 return true;
         return false;
     }
@@ -187,12 +208,16 @@ struct Plan : FusedPlan {
                      : st.type == ST_FUSED4  ? PlanStepView::FUSED4
                      : st.type == ST_FUSED5  ? PlanStepView::FUSED5
                      : st.type == ST_CHANNEL ? PlanStepView::CHANNEL
+                     : st.type == ST_GROUP   ? PlanStepView::GROUP
                                              : PlanStepView::OTHER;
             v.block = (st.type == ST_HERM || st.type == ST_RELABEL || st.type == ST_FUSED4)
                           ? &blocks[st.index]
                           : nullptr;
             v.block5 = st.type == ST_FUSED5 ? &blocks5[st.index] : nullptr;
             v.prim = st.type == ST_CHANNEL ? &prims[st.index] : nullptr;
+            v.group = st.type == ST_GROUP ? &groups[st.index] : nullptr;
+            v.gstages = gstages.data();
+            v.gmats = gmats.data();
             out.push_back(v);
         }
     }
@@ -204,6 +229,8 @@ struct Plan : FusedPlan {
         for (const Step& st : steps) {
             if (st.type == ST_HERM) {
                 b += herm_bytes(nq, blocks[st.index].next_q != 0);
+            } else if (st.type == ST_GROUP) {
+                b += group_bytes(nq, groups[st.index].next_q != 0);
             } else if (st.type == ST_RELABEL || st.type == ST_FUSED4 || st.type == ST_FUSED5) {
                 b += sweep;
             } else if (st.type == ST_CHANNEL) {
@@ -221,6 +248,9 @@ struct Plan : FusedPlan {
         int rc = put(&d_blocks, blocks, stream);
         if (!rc) rc = put(&d_blocks5, blocks5, stream);
         if (!rc) rc = put(&d_stages, stages, stream);
+        if (!rc) rc = put(&d_groups, groups, stream);
+        if (!rc) rc = put(&d_gstages, gstages, stream);
+        if (!rc) rc = put(&d_gmats, gmats, stream);
         return rc ? rc : put(&d_prims, prims, stream);
     }
 
@@ -232,18 +262,24 @@ struct Plan : FusedPlan {
         uint32_t la = 0;
         for (const Step& st : steps) {
             hipError_t e = hipSuccess;
-            if (st.type == ST_HERM || st.type == ST_RELABEL) {
+            if (st.type == ST_HERM || st.type == ST_RELABEL || st.type == ST_GROUP) {
                 if (!re2 || !im2) {
                     set_error("internal: an out-of-place step needs the second pair of planes");
                     return DMX_EINVAL;
                 }
                 const bool h = st.type == ST_HERM;
+                if (st.type == ST_GROUP) {
+                    prof.begin(KC_GROUP, group_bytes(nq, groups[st.index].next_q != 0));
+                    e = launch_group(re, im, re2, im2, d_groups + st.index, d_gstages, d_gmats, nq,
+                                     five(st.index), stream);
+                } else {
                 prof.begin(h ? KC_FUSED4H : KC_RELABEL,
                            h ? herm_bytes(nq, blocks[st.index].next_q != 0) : sweep_bytes);
                 e = h ? launch_fused4_herm(re, im, re2, im2, d_blocks + st.index, nq, max_blocks,
                                            stream, stages_of(st.index))
                       : launch_relabel(re, im, re2, im2, d_blocks + st.index, nq, max_blocks,
                                        stream);
+                }
                 prof.end();
                 std::swap(re, re2);
                 std::swap(im, im2);
@@ -350,10 +386,11 @@ void apply_embedded(std::vector<cd>& U, uint32_t qmask, const std::vector<uint32
 // A block under construction: qubit mask and member gates (circuit indices,
 // in application order).
 struct PB {
-    uint32_t mask;            // qubits of the block's matrix gates
+    uint32_t mask;            // qubits of the block's matrix gates (a group's: all six)
     std::vector<int> gates;
     int dense = -1;           // gates[0, dense) form the matrix, the rest are a trailing
                               // permutation; -1: all of them
+    uint32_t img = 0;         // groups: the qubits on mask's bits after the permutation
 };
 using Seq = std::vector<std::pair<int, int>>;  // (0, index into blocks) or (3, channel gate)
 
@@ -582,10 +619,16 @@ void commute_classes(const Gate& g, uint32_t& zm, uint32_t& xm)
 // their score plus the best score of the block that would follow them; the
 // smaller Q wins ties.  A gate is looked for at most kWindow places past the
 // first ungrouped gate of each qubit.
+//
+// Group sweeps (kmax = six) read runs of as many doubles as the bits that they
+// share with the sweep before span, as those alone can be put lowest: a sweep
+// takes at most kGroupFresh qubits that the one before did not have, so that
+// runs have at least 32 bytes (a lone five-qubit gate may take five).
+constexpr int kGroupFresh = 4;
 class FrontierGrouper {
 public:
     FrontierGrouper(const std::vector<Gate>& circuit, int n, int kmax, bool allow_perm, bool herm)
-        : circuit_(circuit), n_(n), kmax_(kmax), herm_(herm),
+        : circuit_(circuit), n_(n), kmax_(kmax), herm_(herm), group_(kmax == kGroupBits),
           look_(n >= kHermAutoQubits ? kLookDeep : kLook), lists_(n), head_(n, 0),
           mask_(circuit.size(), 0), zm_(circuit.size(), 0), xm_(circuit.size(), 0),
           pos0_(circuit.size(), 0), done_(circuit.size(), 0), mark_(circuit.size(), 0),
@@ -640,6 +683,12 @@ public:
                 pb = PB{0, c.taken};
                 for (int gi : pb.gates) pb.mask |= mask_[gi];
                 touched = pb.mask;
+                if (group_) {  // filled up to six, from the sweep before first
+                    for (uint32_t from : {prev_, ~0u})
+                        for (int q = 0; q < n_ && __builtin_popcount(pb.mask) < kGroupBits; q++)
+                            if ((from >> q) & 1u) pb.mask |= 1u << q;
+                    pb.img = pb.mask;
+                }
                 if (perms) absorb_permutations(pb, touched);
             };
             PB pb;
@@ -658,7 +707,10 @@ public:
                         total += 1L << 40;  // finishes the segment
                     } else {
                         std::vector<Cand> c2;
+                        const uint32_t prev = prev_;
+                        prev_ = cand.img;
                         search(cand.gates, kMaxExplored2, c2);
+                        prev_ = prev;
                         long s2 = 0;
                         for (const Cand& c : c2) s2 = std::max(s2, c.score);
                         total += s2;
@@ -670,6 +722,7 @@ public:
                     }
                 }
             }
+            prev_ = pb.img;
             for (int gi : pb.gates) done_[gi] = 1;
             for (uint32_t b = touched; b; b &= b - 1) {
                 const int q = __builtin_ctz(b);
@@ -808,7 +861,7 @@ private:
     {
         uint32_t qm = pb.mask;
         for (int q = 0; q < n_ && __builtin_popcount(qm) < 4; q++) qm |= 1u << q;
-        if (__builtin_popcount(qm) != 4) return;
+        if (__builtin_popcount(qm) != (group_ ? kGroupBits : 4)) return;
         uint32_t img = qm;
         uint32_t cm = qm;  // super-tile column bits at the default width
         for (int q = 0; q < n_ && __builtin_popcount(cm) < default_tile_bits(n_); q++)
@@ -834,6 +887,7 @@ private:
             }
         }
         if (pb.gates.size() > dense) pb.dense = (int)dense;
+        pb.img = img;
     }
 
     int window_end(int q) const
@@ -979,7 +1033,8 @@ private:
                 ready_on(Q, r);
                 for (int gi : r) {
                     const uint32_t Q2 = Q | mask_[gi];
-                    if (Q2 != Q && __builtin_popcount(Q2) <= limit && !seen.count(Q2))
+                    if (Q2 != Q && __builtin_popcount(Q2) <= limit && !seen.count(Q2) &&
+                        (!group_ || __builtin_popcount(Q2 & ~prev_) <= kGroupFresh))
                         open.push({c.score + weight(gi), Q2, (int)out.size()});
                 }
             }
@@ -1002,6 +1057,9 @@ private:
     const std::vector<Gate>& circuit_;
     const int n_, kmax_;
     const bool herm_;  // trailing gates must keep the block's bits a set of index bits
+    const bool group_;  // blocks are group sweeps on six qubits
+    uint32_t prev_ = 3u;  // groups: the qubits the sweep before leaves on the lowest bits (before
+                          // the first one: the two on bits 0 and 1)
     const int look_;   // candidates compared with the block that would follow them
     std::vector<std::vector<int>> lists_;  // per qubit: its gates in program order
     std::vector<int> head_;                // per qubit: first gate not yet grouped
@@ -1040,6 +1098,20 @@ void group_frontier(const std::vector<Gate>& circuit, int n, int kmax, bool allo
         seg.push_back(gi);
     }
     fg.run(seg, pbs, seq);
+}
+
+// A block of units as a block of the circuit's members.
+void expand_units(const Units& units, PB& pb)
+{
+    std::vector<int> all;
+    int dense = -1;
+    for (size_t t = 0; t < pb.gates.size(); t++) {
+        if ((int)t == pb.dense) dense = (int)all.size();
+        const std::vector<int>& m = units.members[pb.gates[t]];
+        all.insert(all.end(), m.begin(), m.end());
+    }
+    pb.gates.swap(all);
+    pb.dense = dense;
 }
 
 bool has_channel(const std::vector<Gate>& circuit, const std::vector<int>& gates, size_t count)
@@ -1226,6 +1298,127 @@ void build_stages(const std::vector<Gate>& circuit, const std::vector<int>& gate
     }
 }
 
+// A group's stages: what its members do, in order.
+struct StageSpec {
+    uint32_t kind;   // GroupStageKind
+    uint32_t mask;   // the qubits it acts on
+    std::vector<int> members;
+    double cost() const { return kind == GS_UNITARY5 ? 2.0 : kind == GS_PAIR ? 0.5 : 1.0; }  // in 24 MFMAs
+                                                                                            // per 256 entries
+};
+
+// Channel-free members as unitaries of four bits, each member joining the one
+// that must take the fewest new qubits (as in group_least_growth); then every
+// run of them on five qubits that costs more than one unitary of five bits
+// becomes one.
+std::vector<StageSpec> unitary_stages(const std::vector<Gate>& circuit, const std::vector<int>& gates, int n)
+{
+    std::vector<StageSpec> best;
+    double best_cost = 0;
+    std::vector<Gate> sub;
+    for (int gi : gates) sub.push_back(circuit[gi]);
+    for (int attempt = 0; attempt < 3; attempt++) {
+        std::vector<PB> pbs;
+        Seq seq;
+        std::vector<long> w;
+        if (attempt == 0) {
+            group_least_growth(sub, 4, nullptr, pbs, seq);
+        } else {
+            for (const Gate& g : sub) w.push_back(__builtin_popcount(gate_mask(g)) > 1 ? 100 : attempt == 1 ? 1 : 100);
+            group_frontier(sub, n, 4, false, true, nullptr, pbs, seq, &w);
+        }
+        std::vector<StageSpec> out;
+        for (const PB& pb : pbs) {
+            StageSpec sp{__builtin_popcount(pb.mask) > 4 ? GS_UNITARY5 : GS_UNITARY4, pb.mask, {}};
+            for (int i : pb.gates) sp.members.push_back(gates[i]);
+            out.push_back(std::move(sp));
+        }
+        for (size_t i = 0; i < out.size(); i++) {
+            uint32_t mask = 0;
+            double cost = 0;
+            size_t take = i;
+            for (size_t j = i; j < out.size() && __builtin_popcount(mask | out[j].mask) <= 5; j++) {
+                mask |= out[j].mask;
+                cost += out[j].cost();
+                if (cost > 2.0) take = j + 1;
+            }
+            if (take <= i + 1) continue;
+            StageSpec five{GS_UNITARY5, 0u, {}};
+            for (size_t t = i; t < take; t++) {
+                five.mask |= out[t].mask;
+                five.members.insert(five.members.end(), out[t].members.begin(), out[t].members.end());
+            }
+            out.erase(out.begin() + (long)i + 1, out.begin() + (long)take);
+            out[i] = five;
+        }
+        double cost = 0;
+        for (const StageSpec& sp : out) cost += sp.cost();
+        if (attempt == 0 || cost < best_cost) {
+            best.swap(out);
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+// The stages of a group whose first `dense` members are its matrix members.
+// With channels: superoperators of two qubits (a wider gate: a unitary), each
+// member joining the one that must take the fewest new qubits; then each run of
+// channel-free ones becomes unitary_stages where those cost less.
+std::vector<StageSpec> group_stages(const std::vector<Gate>& circuit, const std::vector<int>& gates,
+                                    int dense, int n)
+{
+    const std::vector<int> matrix(gates.begin(), gates.begin() + dense);
+    if (!has_channel(circuit, gates, dense)) return unitary_stages(circuit, matrix, n);
+    std::vector<StageSpec> pairs;
+    std::vector<char> noisy;
+    for (int gi : matrix) {
+        const uint32_t S = gate_mask(circuit[gi]);
+        const int width = __builtin_popcount(S);
+        int first = 0;
+        for (int b = (int)pairs.size() - 1; b >= 0; b--)
+            if (pairs[b].mask & S) {
+                first = b;
+                break;
+            }
+        int best = -1, best_g = 99;
+        for (int b = first; b < (int)pairs.size() && width <= 2; b++) {
+            const int grow = __builtin_popcount(pairs[b].mask | S) - __builtin_popcount(pairs[b].mask);
+            if (pairs[b].kind == GS_PAIR && __builtin_popcount(pairs[b].mask | S) <= 2 && grow <= best_g) {
+                best = b;
+                best_g = grow;
+            }
+        }
+        if (best < 0) {
+            best = (int)pairs.size();
+            pairs.push_back({width <= 2 ? GS_PAIR : width <= 4 ? GS_UNITARY4 : GS_UNITARY5, 0u, {}});
+            noisy.push_back(0);
+        }
+        pairs[best].mask |= S;
+        pairs[best].members.push_back(gi);
+        if (circuit[gi].op == OP_KRAUS) noisy[best] = 1;
+    }
+    std::vector<StageSpec> out;
+    for (size_t i = 0; i < pairs.size();) {
+        std::vector<int> run;
+        double cost = 0, as_unitary = 0;
+        size_t j = i;
+        for (; j < pairs.size() && !noisy[j]; j++) {
+            run.insert(run.end(), pairs[j].members.begin(), pairs[j].members.end());
+            cost += pairs[j].cost();
+        }
+        const std::vector<StageSpec> u = unitary_stages(circuit, run, n);
+        for (const StageSpec& s : u) as_unitary += s.cost();
+        if (as_unitary < cost) {
+            out.insert(out.end(), u.begin(), u.end());
+            i = j;
+        }
+        for (; i < j; i++) out.push_back(pairs[i]);
+        if (i < pairs.size()) out.push_back(pairs[i++]);
+    }
+    return out;
+}
+
 // With a cost model: the grouping the network prices cheapest (defined below
 // with the pricing helpers).
 int choose_grouping(const std::vector<Gate>& circuit, int n, int kmax, bool allow_perm, bool herm,
@@ -1281,18 +1474,8 @@ int plan_blocks(const std::vector<Gate>& circuit, int n, int max_k, BlockPlan& o
         }
     }
     if (grouping) *grouping = which;
-    for (PB& pb : pbs) {  // units -> the circuit's members
-        if (!fold) break;
-        std::vector<int> all_of;
-        int dense = -1;
-        for (size_t t = 0; t < pb.gates.size(); t++) {
-            if ((int)t == pb.dense) dense = (int)all_of.size();
-            const std::vector<int>& m = units->members[pb.gates[t]];
-            all_of.insert(all_of.end(), m.begin(), m.end());
-        }
-        pb.gates.swap(all_of);
-        pb.dense = dense;
-    }
+    for (PB& pb : pbs)
+        if (fold) expand_units(*units, pb);
     const uint32_t all = (1u << n) - 1;
     std::vector<std::pair<int, int>> where(pbs.size());  // pbs index -> order entry
     for (size_t bi = 0; bi < pbs.size(); bi++) {
@@ -1904,13 +2087,244 @@ int reprice_fused5_widths(Plan& plan, int n, CostModel& model)
     return DMX_OK;
 }
 
+// Predicted time of one group sweep with stages of the given cost (StageSpec),
+// base = a four-qubit Hermitian sweep's as the network prices it on the lowest
+// bits.  Fitted at 14 qubits (base 977 us): 1141 us with one stage, 1571 with
+// 2.17 on average, 1600 with 2.41.
+double group_us(double base, double stage_cost)
+{
+    return base * (0.79 + 0.376 * stage_cost);
+}
+
+// Grouping into group sweeps: without a model, the frontier search with its
+// structural scores; with one, the cheapest of that and four other scorings
+// (one-qubit gates weighing 400, 100 and 30, and the gates' predicted unfused
+// times), each searched on a host thread of its own.
+int choose_groups(const std::vector<Gate>& circuit, const std::vector<Gate>& todo, int n,
+                  const Units* units, CostModel* model, std::vector<PB>& pbs, Seq& seq, PlanInfo& pi)
+{
+    constexpr int kCands = 5;
+    std::vector<PB> cand[kCands];
+    Seq cseq[kCands];
+    std::vector<long> w[kCands];
+    double base = 0, us[kCands] = {};
+    if (model) {
+        std::vector<double> gate_us;
+        int rc = unfused_gate_times(todo, n, *model, gate_us);
+        if (rc) return rc;
+        const long one[kCands] = {1, 400, 100, 30, 0};
+        for (int c = 1; c < kCands; c++) {
+            w[c].assign(todo.size(), 1);
+            for (size_t gi = 0; gi < todo.size(); gi++) {
+                const bool multi = __builtin_popcount(gate_mask(todo[gi])) > 1;
+                w[c][gi] = one[c] ? (multi ? 100 : one[c])
+                                  : std::max<long>(1, std::lround(std::min(gate_us[gi], 1e9) * 100.0));
+            }
+        }
+        float f[kMlpFeatures];
+        cost_features(n, CK_HERM, 8, 15u, 0, -1, 0, f);
+        std::vector<float> t;
+        rc = model->price({std::vector<float>(f, f + kMlpFeatures)}, t);
+        if (rc) return rc;
+        base = t[0];
+    }
+    std::exception_ptr err[kCands];
+    std::vector<std::thread> pool;
+    pool.reserve(kCands - 1);
+    auto job = [&](int c) {
+        try {
+            group_frontier(todo, n, kGroupBits, true, true, units, cand[c], cseq[c],
+                           c ? &w[c] : nullptr);
+            for (PB& pb : cand[c]) {
+                if (units) expand_units(*units, pb);  // units -> the circuit's members
+                if (!model) continue;
+                const int dense = pb.dense < 0 ? (int)pb.gates.size() : pb.dense;
+                double cost = 0;
+                for (const StageSpec& sp : group_stages(circuit, pb.gates, dense, n)) cost += sp.cost();
+                us[c] += group_us(base, cost);
+            }
+        } catch (...) {
+            err[c] = std::current_exception();
+        }
+    };
+    for (int c = 1; c < kCands && model; c++) {
+        try {
+            pool.emplace_back([&, c] { job(c); });
+        } catch (const std::system_error&) {
+            job(c);
+        }
+    }
+    job(0);
+    for (std::thread& t : pool) t.join();
+    for (const std::exception_ptr& e : err)
+        if (e) std::rethrow_exception(e);
+    int which = 0;
+    for (int c = 1; c < kCands && model; c++)
+        if (us[c] < us[which]) which = c;
+    pi.greedy_us = us[0];
+    pi.predicted_us = us[which];
+    pi.grouping = which == 0 ? 1u : which == 1 ? 5u : which == 4 ? 2u : 4u;
+    pbs.swap(cand[which]);
+    seq.swap(cseq[which]);
+    return DMX_OK;
+}
+
+// The plan of a circuit as group sweeps (six qubits each, stages of at most
+// four, or five for a gate that wide) and a relabelling home at the end.
+// Each sweep is written with its qubits (after its trailing index map) on bits
+// 0..5, those that the next sweep shares lowest.
+int build_group_plan(const std::vector<Gate>& circuit, int n, CostModel* model, FusedPlan** out,
+                     PlanInfo* info)
+{
+    PlanInfo pi;
+    bool channels = false;
+    for (const Gate& g : circuit) channels = channels || g.op == OP_KRAUS;
+    std::unique_ptr<Units> units;
+    if (channels) units.reset(new Units(circuit));
+    const std::vector<Gate>& todo = channels ? units->gates : circuit;
+    std::vector<PB> pbs;
+    Seq seq;
+    int rc = choose_groups(circuit, todo, n, units.get(), model, pbs, seq, pi);
+    if (rc) return rc;
+    std::unique_ptr<Plan> plan(new Plan());
+    plan->n = n;
+    plan->channels_inside = channels;
+    BitOrder bo(n);
+    auto move_bits = [&](const std::vector<int>& to, uint32_t v) {
+        uint32_t o = 0;
+        for (int q = 0; q < n; q++)
+            if ((v >> q) & 1u) o |= 1u << to[q];
+        return o;
+    };
+    for (size_t i = 0; i < pbs.size(); i++) {
+        const PB& pb = pbs[i];
+        GroupBlock b;
+        std::memset(&b, 0, sizeof(b));
+        b.qmask = bo.phys(pb.mask);
+        if (__builtin_popcount(pb.mask) != kGroupBits || __builtin_popcount(pb.img) != kGroupBits ||
+            !(b.qmask & 1u)) {
+            set_error("internal: a group sweep needs six qubits, one of them on bit 0");
+            return DMX_EINVAL;
+        }
+        b.stage0 = (uint32_t)plan->gstages.size();
+        auto local = [&](int q) {  // local bit of logical qubit q
+            return (uint32_t)__builtin_popcount(b.qmask & ((1u << bo.sigma[q]) - 1u));
+        };
+        const int dense = pb.dense < 0 ? (int)pb.gates.size() : pb.dense;
+        for (const StageSpec& sp : group_stages(circuit, pb.gates, dense, n)) {
+            GroupStage st;
+            std::memset(&st, 0, sizeof(st));
+            st.kind = sp.kind;
+            st.mat = (uint32_t)plan->gmats.size();
+            const int width = sp.kind == GS_PAIR ? 2 : sp.kind == GS_UNITARY4 ? 4 : 5;
+            uint32_t mask = sp.mask;
+            for (uint32_t m = pb.mask; __builtin_popcount(mask) < width; m &= m - 1) mask |= m & (~m + 1);
+            int at = 0;
+            for (uint32_t set : {mask, pb.mask & ~mask})
+                for (uint32_t m = set; m; m &= m - 1) st.bits |= local(__builtin_ctz(m)) << (4 * at++);
+            const std::vector<cd> M = sp.kind == GS_PAIR
+                                          ? pair_superoperator(circuit, sp.members, mask)
+                                          : product_of(circuit, sp.members.data(), sp.members.size(), mask);
+            for (const cd& v : M) plan->gmats.push_back(v.real());
+            for (const cd& v : M) plan->gmats.push_back(v.imag());
+            plan->gstages.push_back(st);
+        }
+        b.stages = (uint32_t)plan->gstages.size() - b.stage0;
+        b.mat_end = (uint32_t)plan->gmats.size();
+        // the output order
+        uint32_t Lp[16];
+        trailing_linear(circuit, pb, n, Lp);
+        uint32_t bp = 0;
+        for (size_t t = dense; t < pb.gates.size(); t++) {  // pi(0)
+            const Gate& g = circuit[pb.gates[t]];
+            const uint32_t x = g.qb[0], y = g.qb[1];
+            if (g.op == OP_X) {
+                bp ^= 1u << x;
+            } else if (g.op == OP_CX) {
+                bp ^= ((bp >> x) & 1u) << y;
+            } else {
+                const uint32_t d = ((bp >> x) ^ (bp >> y)) & 1u;
+                bp ^= (d << x) | (d << y);
+            }
+        }
+        const uint32_t next = i + 1 < pbs.size() ? pbs[i + 1].mask : 0u;
+        std::vector<int> order;
+        std::vector<char> placed(n, 0);
+        auto place = [&](int q) {
+            if (!placed[q]) order.push_back(q);
+            placed[q] = 1;
+        };
+        for (uint32_t set : {pb.img & next, pb.img})
+            for (uint32_t m = set; m; m &= m - 1) place(__builtin_ctz(m));
+        for (int p = 0; p < n; p++) place(bo.sinv[p]);
+        BitOrder nb(n);
+        for (int k = 0; k < n; k++) {
+            nb.sigma[order[k]] = k;
+            nb.sinv[k] = order[k];
+        }
+        for (int p = 0; p < n; p++) b.perm_L[p] = move_bits(nb.sigma, Lp[bo.sinv[p]]);
+        b.perm_b = move_bits(nb.sigma, bp);
+        b.next_q = nb.phys(next);
+        // f on local indices and its inverse
+        uint32_t f[6];
+        {
+            int t = 0;
+            for (uint32_t m = b.qmask; m; m &= m - 1) f[t++] = b.perm_L[__builtin_ctz(m)];
+        }
+        for (uint32_t a = 0; a < 64; a++) {
+            uint32_t y = 0;
+            for (int t = 0; t < 6; t++)
+                if ((a >> t) & 1u) y ^= f[t];
+            if (y >= 64) {
+                set_error("internal: a group's index map leaves its bits");
+                return DMX_EINVAL;
+            }
+            if ((y & (y - 1)) == 0 && y) b.finv[__builtin_ctz(y)] = a;
+        }
+        plan->steps.push_back({ST_GROUP, (int)plan->groups.size(), 0});
+        plan->groups.push_back(b);
+        pi.herm_blocks++;
+        pi.fused_blocks++;
+        pi.perm_blocks += dense < (int)pb.gates.size() ? 1 : 0;
+        pi.tile_hist[8]++;
+        bo = nb;
+    }
+    if (!bo.home()) {
+        FusedBlock fb;
+        std::memset(&fb, 0, sizeof(fb));
+        fb.perm_on = 1;
+        for (int p = 0; p < n; p++) fb.perm_L[p] = 1u << bo.sinv[p];
+        plan->steps.push_back({ST_RELABEL, (int)plan->blocks.size(), 0});
+        plan->blocks.push_back(fb);
+        pi.relabels++;
+    }
+    *out = plan.release();
+    if (info) *info = pi;
+    return DMX_OK;
+}
+
 }  // namespace
+
+bool group_wanted(const std::vector<Gate>& circuit, int n)
+{
+    bool channels = false, wide = false;
+    for (const Gate& g : circuit) {
+        channels = channels || g.op == OP_KRAUS;
+        wide = wide || __builtin_popcount(gate_mask(g)) > 4;
+    }
+    return (channels && n >= 12) || (wide && n >= 13);
+}
 
 int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model,
                      int tile_bits, bool allow_perm, FusedPlan** out, PlanInfo* info, bool herm,
-                     bool fold)
+                     bool fold, bool group)
 {
     *out = nullptr;
+    if (group && herm && allow_perm && fold && n >= kHermMinQubits && n <= 16) {
+        bool linear = !circuit.empty();
+        for (const Gate& g : circuit) linear = linear && g.op != OP_SRN;
+        if (linear) return build_group_plan(circuit, n, tile_bits > 0 ? nullptr : model, out, info);
+    }
     PlanInfo pi;
     BlockPlan bp;
     bool fusable = false;
@@ -1936,6 +2350,7 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
     plan->blocks = std::move(bp.blocks);
     plan->blocks5 = std::move(bp.blocks5);
     plan->stages = std::move(bp.stages);
+    plan->channels_inside = !plan->stages.empty();
     for (const auto& o : bp.order) {
         if (o.first == 3) {
             const int first = (int)plan->prims.size();

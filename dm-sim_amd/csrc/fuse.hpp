@@ -9,6 +9,7 @@
 #include "lower.hpp"
 #include "prim.hpp"
 #include "fused.hpp"
+#include "group.hpp"
 #include "prof.hpp"
 
 namespace dmx {
@@ -35,11 +36,14 @@ struct PlanInfo {
 
 // One step of a fused plan as the executor runs it (host-side checks).
 struct PlanStepView {
-    enum Kind { FUSED4, FUSED5, HERM, RELABEL, CHANNEL, OTHER } kind;
+    enum Kind { FUSED4, FUSED5, HERM, RELABEL, CHANNEL, OTHER, GROUP } kind;
     const FusedBlock* block;    // FUSED4, HERM, RELABEL: its record as launched
     const FusedBlock5* block5;  // FUSED5
     const PrimOp* prim;         // CHANNEL: its record for the stored orientation (the
                                 // conj-transposed one follows it)
+    const GroupBlock* group;    // GROUP, with the plan's stages and matrices
+    const GroupStage* gstages;
+    const double* gmats;
 };
 
 // Algorithmic bytes of one Hermitian block sweep (k_fused4_herm) on n >= 8
@@ -160,9 +164,24 @@ inline bool permuting_pays(int n, double sweeps, double permuting, double sweeps
 // sweeps (k_fused4_herm) with rho's index bits relabelled so that each
 // block's output lands in aligned 16-column runs; rho returns to the
 // circuit's bit order (k_relabel) before any other step and at the end.
+// group (with herm and fold): the whole plan as group sweeps (k_group) of six
+// qubits whose stages are the blocks: several blocks of at most four qubits
+// (five for a five-qubit gate or where it costs less) to a sweep.
 int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model,
                      int tile_bits, bool allow_perm, FusedPlan** out, PlanInfo* info,
-                     bool herm = false, bool fold = false);
+                     bool herm = false, bool fold = false, bool group = false);
+
+// Whether a circuit's Hermitian plan runs as group sweeps.  With channels, from
+// 12 qubits: a group holds their whole neighbourhood where a four-qubit block
+// with a channel on every gate fills up with channels (a 300-member 12-qubit
+// circuit 1680 -> 1315 us; below 12 qubits rho fits the caches and a sweep costs
+// its launch).  With five-qubit gates, from 13: the five-qubit sweep has no
+// Hermitian form (structured circuits 20.3 -> 14.3 ms at 13 qubits, 77 -> 62.5
+// at 14, 332 -> 289 at 15).  Other unitary circuits keep four-qubit sweeps: on
+// 2130 gates at 14 qubits 116 group sweeps of 1.57 ms take 182 ms, 181 of the
+// others 177, as a group's 2.2 stages occupy the matrix cores for 1.15 ms that
+// overlap its 1.1 ms of memory traffic only in part.
+bool group_wanted(const std::vector<Gate>& circuit, int n);
 
 // From this many qubits the engine folds channels into blocks.  A noisy
 // 318-member circuit at 8 qubits takes 9 sweeps instead of 138 and 180 channel

@@ -19,6 +19,7 @@ enum KernelClass : int {
     KC_FUSED4H,       // k_fused4_herm: a 4-qubit block on the upper tiles of Hermitian rho, out of place
     KC_RELABEL,       // k_relabel: rho's index bits relabelled, out of place
     KC_TRANSPOSE,     // k_conj_transpose, in place
+    KC_GROUP,         // k_group: blocks on up to six qubits on the upper tiles of Hermitian rho, out of place
     KC_COUNT
 };
 
