@@ -161,11 +161,14 @@ int Engine::upload()
         // no plan (SRN in the circuit, or n < 4): the run uses the plain sweeps
         const bool herm = herm_wanted();
         const bool fold = n_ >= kFoldChannelQubits;
+        // the settings that ask for a form of sweep keep the sweeps
+        const bool resident = fusion_permute_ && fusion_herm_ == 1 && tile_bits_ == 0 &&
+                              resident_wanted(circuit_, n_, fusion_max_k_);
         int rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_,
                                   fusion_permute_, &plan_, &plan_info_, herm, fold,
-                                  group_wanted(circuit_, n_));
+                                  group_wanted(circuit_, n_), resident);
         if (rc) return rc;
-        if (plan_ && plan_info_.perm_blocks > 0 && n_ < kPermuteSureQubits && fusion_herm_ != 2) {
+        if (plan_ && !plan_->resident() && plan_info_.perm_blocks > 0 && n_ < kPermuteSureQubits && fusion_herm_ != 2) {
             // a short sweep is latency-bound and a permuting one pays its index
             // map's set-up: keep the permuting plan only if it still wins
             FusedPlan* inplace = nullptr;
@@ -207,7 +210,8 @@ int Engine::upload()
             rc = plan_->upload(stream_);
             if (rc) return rc;
             tuned_tile_bits_ = 0;
-            if (!model_ && tile_bits_ == 0 && fusion_autotune_ && plan_info_.herm_blocks == 0) {
+            if (!model_ && tile_bits_ == 0 && fusion_autotune_ && plan_info_.herm_blocks == 0 &&
+                !plan_->resident()) {
                 // the greedy plan's tile width, measured: on the second pair of
                 // planes if there is one, else on scratch planes (rho untouched)
                 double *sr = d_re2_, *si = d_im2_;
@@ -417,7 +421,7 @@ int Engine::run_fused()
         // launch-bound at small n: one graph launch instead of one per step
         RunGraph* rg = nullptr;
         for (RunGraph& g : graphs_)
-            if (g.exec && g.transposed == transposed_ && g.re == d_re_ && g.im == d_im_) rg = &g;
+            if (g.exec && (g.transposed == transposed_ || plan_->resident()) && g.re == d_re_ && g.im == d_im_) rg = &g;
         if (!rg) {
             RunGraph& g = graphs_[graph_next_];
             graph_next_ ^= 1;
@@ -450,6 +454,7 @@ int Engine::run_fused()
         d_im_ = rg->im_end;
         d_re2_ = rg->re2_end;
         d_im2_ = rg->im2_end;
+        transposed_ = transposed_ != plan_->flips();
         float ms = 0.f;
         HIPTRY(hipEventElapsedTime(&ms, ev0_, ev1_));
         last_ms_ = ms;
@@ -462,6 +467,7 @@ int Engine::run_fused()
     int rc = plan_->execute(d_re_, d_im_, d_re2_, d_im2_, n_, transposed_, stream_, prof_,
                             &last_launches_, &last_sweeps_);
     if (rc) return rc;
+    transposed_ = transposed_ != plan_->flips();
     HIPTRY(hipEventRecord(ev1_, stream_));
     HIPTRY(hipEventSynchronize(ev1_));
     float ms = 0.f;

@@ -34,6 +34,7 @@
 #include "fused.hpp"
 #include "group.hpp"
 #include "mlp.hpp"
+#include "resident.hpp"
 #include "sweep.hpp"
 
 namespace dmx {
@@ -84,6 +85,8 @@ struct Plan : FusedPlan {
     std::vector<GroupBlock> groups;
     std::vector<GroupStage> gstages;
     std::vector<double> gmats;
+    std::vector<ResidentPart> rparts;  // resident plans: every step's block
+    ResidentEnd rend = {};
     bool channels_inside = false;  // a block or group holds channels
     std::vector<PrimOp> prims;
     std::vector<Step> steps;
@@ -93,6 +96,7 @@ struct Plan : FusedPlan {
     GroupBlock* d_groups = nullptr;
     GroupStage* d_gstages = nullptr;
     double* d_gmats = nullptr;
+    ResidentPart* d_rparts = nullptr;
     PrimOp* d_prims = nullptr;
     int max_blocks = kFusedGridCap;
 
@@ -104,6 +108,7 @@ struct Plan : FusedPlan {
         if (d_groups) (void)hipFree(d_groups);
         if (d_gstages) (void)hipFree(d_gstages);
         if (d_gmats) (void)hipFree(d_gmats);
+        if (d_rparts) (void)hipFree(d_rparts);
         if (d_prims) (void)hipFree(d_prims);
     }
 
@@ -132,6 +137,18 @@ struct Plan : FusedPlan {
 
     bool staged() const override { return channels_inside; }
 
+    // Every block on resident rows (plans of nothing but four-qubit blocks).
+    void make_resident()
+    {
+        std::vector<int> order;
+        for (const Step& st : steps) order.push_back(st.index);
+        if (!order.empty()) build_resident(blocks, order, n, rparts, rend);
+    }
+
+    bool resident() const override { return !rparts.empty(); }
+
+    bool flips() const override { return !rparts.empty() && n > kResidentColumnQubits; }
+
     bool five(int group) const
     {
         const GroupBlock& b = groups[group];
@@ -142,6 +159,7 @@ struct Plan : FusedPlan {
 
     bool needs_alt() const override
     {
+        if (!rparts.empty()) return false;
         for (const Step& st : steps)
             if ((st.type == ST_FUSED4 && blocks[st.index].perm_on) || st.type == ST_HERM ||
                 st.type == ST_RELABEL || st.type == ST_GROUP)
@@ -225,6 +243,7 @@ struct Plan : FusedPlan {
     double bytes(int nq) const override
     {
         const double sweep = 32.0 * (double)(1ull << (2 * nq));
+        if (!rparts.empty()) return (flips() ? 3.0 : 2.0) * sweep;
         double b = 0;
         for (const Step& st : steps) {
             if (st.type == ST_HERM) {
@@ -251,6 +270,7 @@ struct Plan : FusedPlan {
         if (!rc) rc = put(&d_groups, groups, stream);
         if (!rc) rc = put(&d_gstages, gstages, stream);
         if (!rc) rc = put(&d_gmats, gmats, stream);
+        if (!rc) rc = put(&d_rparts, rparts, stream);
         return rc ? rc : put(&d_prims, prims, stream);
     }
 
@@ -260,6 +280,31 @@ struct Plan : FusedPlan {
     {
         const double sweep_bytes = 32.0 * (double)(1ull << (2 * nq));
         uint32_t la = 0;
+        if (!rparts.empty()) {
+            hipError_t e = hipSuccess;
+            auto launch = [&](int cls, auto&& f) {
+                if (e != hipSuccess) return;
+                prof.begin(cls, sweep_bytes);
+                e = f();
+                prof.end();
+                la++;
+            };
+            auto pass = [&](bool slow) {
+                launch(KC_RESIDENT, [&] {
+                    return launch_resident(re, im, d_rparts, (int)steps.size(), rend, nq, slow, stream);
+                });
+            };
+            pass(false);
+            if (flips()) launch(KC_TRANSPOSE, [&] { return launch_conj_transpose(re, im, nq, stream); });
+            pass(!flips());
+            if (e != hipSuccess) {
+                set_error(std::string("resident run launch: ") + hipGetErrorString(e));
+                return DMX_EHIP;
+            }
+            *launches = la;
+            *sweeps = la;
+            return DMX_OK;
+        }
         for (const Step& st : steps) {
             hipError_t e = hipSuccess;
             if (st.type == ST_HERM || st.type == ST_RELABEL || st.type == ST_GROUP) {
@@ -2305,6 +2350,14 @@ int build_group_plan(const std::vector<Gate>& circuit, int n, CostModel* model, 
 
 }  // namespace
 
+bool resident_wanted(const std::vector<Gate>& circuit, int n, int max_k)
+{
+    if (n < 4 || n > kResidentMaxQubits || max_k > 4) return false;
+    for (const Gate& g : circuit)
+        if (g.op == OP_KRAUS || g.op == OP_SRN || __builtin_popcount(gate_mask(g)) > 4) return false;
+    return true;
+}
+
 bool group_wanted(const std::vector<Gate>& circuit, int n)
 {
     bool channels = false, wide = false;
@@ -2317,7 +2370,7 @@ bool group_wanted(const std::vector<Gate>& circuit, int n)
 
 int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model,
                      int tile_bits, bool allow_perm, FusedPlan** out, PlanInfo* info, bool herm,
-                     bool fold, bool group)
+                     bool fold, bool group, bool resident)
 {
     *out = nullptr;
     if (group && herm && allow_perm && fold && n >= kHermMinQubits && n <= 16) {
@@ -2344,6 +2397,8 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
         if (rc) return rc;
         rc = choose_fused5(circuit, n, bp, *model, sub, pi);
         if (rc) return rc;
+        if (resident)  // no block as primitive sweeps, whatever these would take
+            for (auto& p : plain) p.clear();
     }
     Plan* plan = new Plan();
     plan->n = n;
@@ -2388,6 +2443,7 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
             plan->steps.push_back({ST_PLAIN, first, (int)plan->prims.size() - first});
         }
     }
+    if (resident) plan->make_resident();
     if (herm) to_hermitian(*plan, n, pi);
     if (herm && model && tile_bits <= 0) {
         rc = reprice_fused5_widths(*plan, n, *model);

@@ -66,6 +66,10 @@ struct FusedPlan {
     // Whether blocks hold channels (FusedStage): execute then takes rho in its
     // stored orientation only (transposed = false).
     virtual bool staged() const = 0;
+    // Whether every block runs on resident rows (resident.hpp) instead of in sweeps.
+    virtual bool resident() const = 0;
+    // Whether execute leaves rho in the other orientation (conj-transposed).
+    virtual bool flips() const = 0;
     // Whether execute needs a second pair of planes (blocks with a trailing
     // permutation run out of place).
     virtual bool needs_alt() const = 0;
@@ -167,9 +171,17 @@ inline bool permuting_pays(int n, double sweeps, double permuting, double sweeps
 // group (with herm and fold): the whole plan as group sweeps (k_group) of six
 // qubits whose stages are the blocks: several blocks of at most four qubits
 // (five for a five-qubit gate or where it costs less) to a sweep.
+// resident (where resident_wanted, with allow_perm): the blocks run on resident
+// rows; the model's prices still are those of sweeps.
 int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model,
                      int tile_bits, bool allow_perm, FusedPlan** out, PlanInfo* info,
-                     bool herm = false, bool fold = false, bool group = false);
+                     bool herm = false, bool fold = false, bool group = false,
+                     bool resident = false);
+
+// Whether a unitary circuit's blocks may run on resident rows: 4 to
+// kResidentMaxQubits qubits, no channels, no gate on more than four qubits, and at
+// most four qubits to a block.
+bool resident_wanted(const std::vector<Gate>& circuit, int n, int max_k);
 
 // Whether a circuit's Hermitian plan runs as group sweeps.  With channels, from
 // 12 qubits: a group holds their whole neighbourhood where a four-qubit block

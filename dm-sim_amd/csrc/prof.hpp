@@ -20,6 +20,7 @@ enum KernelClass : int {
     KC_RELABEL,       // k_relabel: rho's index bits relabelled, out of place
     KC_TRANSPOSE,     // k_conj_transpose, in place
     KC_GROUP,         // k_group: blocks on up to six qubits on the upper tiles of Hermitian rho, out of place
+    KC_RESIDENT,      // k_resident: every fused block on one index, whole rows resident
     KC_COUNT
 };
 

@@ -1,0 +1,186 @@
+// resident.hip -- fused four-qubit blocks on whole rows of rho, for gfx950.
+//
+// Rows do not depend on each other on the column index, so a workgroup loads
+// whole rows (2^n entries, 4 KiB to 32 KiB) into LDS once, applies every block of
+// the circuit to their columns with FP64 MFMA and stores them once; a second pass
+// does the same to the row index.  A block sweep, one launch per block, moves rho
+// through the caches each time and pays a launch: 6 us at 8 qubits and 38 us at 11.
+//
+// A block is Y = U X on the 16 x 16 tiles of the rows, X's columns the other index
+// bits: a lane reads and writes the same four places, so a block takes one barrier
+// (none where a wave holds the row, up to 8 qubits).  Index permutations between
+// blocks (X, CX, SWAP) only change the places that later records name.
+#include <hip/hip_runtime.h>
+
+#include "resident.hpp"
+
+namespace dmx {
+
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ d4 mfma(double a, double b, d4 c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+}  // namespace
+
+// n <= LOGE; a chunk is 2^LOGE entries, 2^(LOGE - 8) tiles, dealt to the waves
+// in runs.  SLOW: rows and columns of rho exchanged, and conjugated values.
+template <int LOGE, int WAVES, bool SLOW>
+__global__ void __launch_bounds__(64 * WAVES, 4)
+    k_resident(double* __restrict__ re, double* __restrict__ im, const double2* __restrict__ parts,
+               int blocks, ResidentEnd end, int n)
+{
+    constexpr int kThreads = 64 * WAVES;
+    constexpr int kPer = (1 << (LOGE - 8)) / WAVES;  // tiles of a wave
+    __shared__ double2 s[1 << LOGE];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u, wave = tid >> 6;
+    // entry i of the thread's share in memory order: its index in the chunk, its offset
+    auto entry = [&](uint32_t i, uint32_t& e) -> uint64_t {
+        const uint32_t f = SLOW ? tid + i * kThreads : 2 * (tid + i * kThreads);
+        if constexpr (!SLOW) {
+            e = f;
+            return ((uint64_t)blockIdx.x << LOGE) + f;
+        }
+        const int rows = LOGE - n;  // 2^rows columns of rho to a chunk, neighbours together
+        const uint32_t c = f & ((1u << rows) - 1u), r = f >> rows;
+        e = r | c << n;
+        return ((uint64_t)r << n) + ((uint64_t)blockIdx.x << rows) + c;
+    };
+
+    const double2* src = parts + lane;
+    double2 next[kResidentParts];
+#pragma unroll
+    for (int i = 0; i < kResidentParts; i++) next[i] = src[64 * i];
+
+    if constexpr (SLOW) {
+#pragma unroll
+        for (int i = 0; i < (1 << LOGE) / kThreads; i++) {
+            uint32_t e;
+            const uint64_t off = entry(i, e);
+            s[row_place(e, 3, LOGE)] = make_double2(re[off], -im[off]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < (1 << LOGE) / kThreads / 2; i++) {
+            uint32_t e;
+            const uint64_t off = entry(i, e);
+            const double2 r = *reinterpret_cast<const double2*>(re + off);
+            const double2 m = *reinterpret_cast<const double2*>(im + off);
+            const uint32_t x = row_place(e, 3, LOGE);
+            s[x] = make_double2(r.x, m.x);
+            s[x ^ 1u] = make_double2(r.y, m.y);
+        }
+    }
+
+    for (int b = 0; b < blocks; b++) {
+        const double ur[4] = {next[0].x, next[0].y, next[1].x, next[1].y};
+        const double ui[4] = {next[2].x, next[2].y, next[3].x, next[3].y};
+        const uint32_t w0 = (uint32_t)__double2loint(next[4].x), w1 = (uint32_t)__double2hiint(next[4].x);
+        const uint32_t w2 = (uint32_t)__double2loint(next[4].y);
+        const uint32_t c0 = w0 >> 16, c1 = w1 & 0xFFFFu;
+        const uint32_t t[3] = {w1 >> 16, w2 & 0xFFFFu, w2 >> 16};
+        uint32_t x[kPer][4];
+#pragma unroll
+        for (int u = 0; u < kPer; u++) {
+            const uint32_t tile = wave * kPer + u;
+            uint32_t base = w0 & 0xFFFFu;
+#pragma unroll
+            for (int i = 0; i < LOGE - 8; i++) base ^= (tile >> i) & 1u ? t[i] : 0u;
+            x[u][0] = base;
+            x[u][1] = base ^ c0;
+            x[u][2] = base ^ c1;
+            x[u][3] = base ^ c0 ^ c1;
+        }
+        src += 64 * kResidentParts;
+        __syncthreads();
+        if (b + 1 < blocks) {
+#pragma unroll
+            for (int i = 0; i < kResidentParts; i++) next[i] = src[64 * i];
+        }
+        double2 v[kPer][4];
+#pragma unroll
+        for (int u = 0; u < kPer; u++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[u][c] = s[x[u][c]];
+        // three real products, the additions left to the accumulators: with
+        // K = Ur (Xr + Xi), re = K - (Ur + Ui) Xi and im = K + (Ui - Ur) Xr
+        d4 yr[kPer], yi[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; u++) yr[u] = d4{0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int u = 0; u < kPer; u++) yr[u] = mfma(ur[c], v[u][c].x + v[u][c].y, yr[u]);
+#pragma unroll
+        for (int u = 0; u < kPer; u++) yi[u] = yr[u];
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int u = 0; u < kPer; u++) {
+                yr[u] = mfma(-ur[c] - ui[c], v[u][c].y, yr[u]);
+                yi[u] = mfma(ui[c] - ur[c], v[u][c].x, yi[u]);
+            }
+#pragma unroll
+        for (int u = 0; u < kPer; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) s[x[u][r]] = make_double2(yr[u][r], yi[u][r]);
+    }
+    __syncthreads();
+
+    auto end_place = [&](uint32_t e) {
+        uint32_t x = end.base;
+#pragma unroll
+        for (int i = 0; i < LOGE; i++) x ^= (e >> i) & 1u ? end.bit[i] : 0u;
+        return x;
+    };
+    if constexpr (SLOW) {
+#pragma unroll
+        for (int i = 0; i < (1 << LOGE) / kThreads; i++) {
+            uint32_t e;
+            const uint64_t off = entry(i, e);
+            const double2 v = s[end_place(e)];
+            re[off] = v.x;
+            im[off] = -v.y;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < (1 << LOGE) / kThreads / 2; i++) {
+            uint32_t e;
+            const uint64_t off = entry(i, e);
+            const uint32_t x = end_place(e);
+            const double2 a = s[x], b = s[x ^ end.bit[0]];
+            *reinterpret_cast<double2*>(re + off) = make_double2(a.x, b.x);
+            *reinterpret_cast<double2*>(im + off) = make_double2(a.y, b.y);
+        }
+    }
+}
+
+hipError_t launch_resident(double* re, double* im, const ResidentPart* d_parts, int blocks,
+                           const ResidentEnd& end, int n, bool slow, hipStream_t stream)
+{
+    if (n < 4 || n > (slow ? kResidentColumnQubits : kResidentMaxQubits) || blocks < 1)
+        return hipErrorInvalidValue;
+    const unsigned grid = 1u << (2 * n - resident_log_entries(n));
+    const double2* p = reinterpret_cast<const double2*>(d_parts);
+    if (slow) {
+        if (n <= 8)
+            k_resident<8, 1, true><<<grid, 64, 0, stream>>>(re, im, p, blocks, end, n);
+        else
+            k_resident<9, 2, true><<<grid, 128, 0, stream>>>(re, im, p, blocks, end, n);
+        return hipGetLastError();
+    }
+    switch (n <= 8 ? 8 : n) {
+    case 8: k_resident<8, 1, false><<<grid, 64, 0, stream>>>(re, im, p, blocks, end, n); break;
+    case 9: k_resident<9, 2, false><<<grid, 128, 0, stream>>>(re, im, p, blocks, end, n); break;
+    case 10: k_resident<10, 4, false><<<grid, 256, 0, stream>>>(re, im, p, blocks, end, n); break;
+    default: k_resident<11, 8, false><<<grid, 512, 0, stream>>>(re, im, p, blocks, end, n); break;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace dmx

@@ -1,0 +1,59 @@
+// resident.hpp -- fused blocks on whole rows of rho held in LDS (resident.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <vector>
+
+#include "fused.hpp"
+#include "rows.hpp"
+
+namespace dmx {
+
+// Largest n that runs resident (a row of 2048 entries is 32 KiB, so five
+// workgroups fit a CU).  From 12 qubits the Hermitian sweeps, which transform half
+// of rho, are the default.
+constexpr int kResidentMaxQubits = 11;
+// Up to this many qubits the second pass reads and writes columns itself, as
+// rho (4 MiB) stays in the caches; above, a conjugate transpose stands between two
+// row passes, and rho is held conj-transposed after the run.
+constexpr int kResidentColumnQubits = 9;
+
+// A workgroup's chunk: 2^L entries of rho, whole rows (the low n bits of an entry
+// number its column, the others its row).
+inline int resident_log_entries(int n) { return n > 8 ? n : 8; }
+
+// One block as a wave reads it: part s of lane l at [s * 64 + l].  Lane l =
+// i + 16 k holds row i of the 16 x 16 matrix: u[0..1] the real parts of columns
+// k, 4 + k and 8 + k, 12 + k, u[2..3] the imaginary ones.  LDS places (row_place)
+// compose by XOR: at for the lane, c0 and c1 for the bits of the matrix index that
+// the chunk c of four columns numbers, t0, t1, t2 for the bits of the tile's number.
+// The lane reads entries (4 c + k) and writes them: the same places.
+struct ResidentPart {
+    union {
+        double u[2];
+        struct {
+            uint16_t at, c0, c1, t0, t1, t2, pad[2];
+        } place;
+    };
+};
+constexpr int kResidentParts = 5;  // four of the matrix, then the places
+
+// The last record: the place of entry 0 and, bit by bit, of an entry's index,
+// for the store.
+struct ResidentEnd {
+    uint32_t base;
+    uint32_t bit[11];
+};
+
+// The records of a sequence of blocks.  A block's trailing permutation costs
+// nothing: it changes which places the index bits mean from there on.
+void build_resident(const std::vector<FusedBlock>& blocks, const std::vector<int>& order, int n,
+                    std::vector<ResidentPart>& parts, ResidentEnd& end);
+
+// rho <- rho U^T for the product U of all blocks, 4 <= n <= kResidentMaxQubits;
+// slow (n <= kResidentColumnQubits): rho <- conj(U) rho.  In place.
+hipError_t launch_resident(double* re, double* im, const ResidentPart* d_parts, int blocks,
+                           const ResidentEnd& end, int n, bool slow, hipStream_t stream);
+
+}  // namespace dmx
