@@ -126,12 +126,15 @@ struct BlockPlan {
 // cheaper of its fused sweep and its gates unfused); without a model the one
 // with fewer sweeps of the first two.  *grouping (may be null) = the choice:
 // 0..5 in that order.
+// resident: the blocks run on resident rows, all at one price: of the first two
+// groupings the one with fewer blocks, whatever the model, and any X, CX or SWAP
+// may trail a block.
 // fold: a channel is a member of a block like a one-qubit gate, and a block
 // with channels runs as stages (unless a gate is wider than four qubits:
 // channels then stand between blocks, as without fold).
 int plan_blocks(const std::vector<Gate>& circuit, int n, int max_k, BlockPlan& out, bool& fusable,
                 bool allow_perm = false, bool herm = false, CostModel* model = nullptr,
-                uint32_t* grouping = nullptr, bool fold = false);
+                uint32_t* grouping = nullptr, bool fold = false, bool resident = false);
 
 // Relative extra cost of a sweep with a trailing permutation on n qubits:
 // about 2.5 us of index-map set-up against the sweep's own time (32 * 4^n bytes

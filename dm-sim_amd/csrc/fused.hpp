@@ -11,7 +11,7 @@ namespace dmx {
 // (trailing X, CX and SWAP gates): when perm_on, entry (i, j) of U rho U^dagger
 // goes to (pi(i), pi(j)) with pi(x) = L x + b over GF(2), L given by its
 // columns perm_L[q] = the image of bit q (q < n), and the sweep writes into a
-// second pair of planes.  pi leaves bit 0 in place (perm_L[0] = 1).
+// second pair of planes.  In a sweep pi leaves bit 0 in place (perm_L[0] = 1).
 struct FusedBlock {
     uint32_t qmask;  // exactly four qubits
     uint32_t m;      // super-tile column bits (the tile schedule), see tile_bits_ok
