@@ -16,6 +16,7 @@
 
 #include "dmsim_amd.h"
 #include "engine.hpp"
+#include "sweep.hpp"
 
 namespace dmx {
 
@@ -45,10 +46,12 @@ void Batch::free_device()
     graph_ = nullptr;
     for (void* p : {(void*)pool_, (void*)pool_alt_, (void*)d_blocks_, (void*)d_entries_,
                     (void*)d_re_off_, (void*)d_terms_, (void*)d_jobs_, (void*)d_energy_,
-                    (void*)d_diag_, (void*)d_diag_off_})
+                    (void*)d_diag_, (void*)d_diag_off_, (void*)d_res_jobs_, (void*)d_res_parts_})
         if (p) (void)hipFree(p);
     d_diag_ = nullptr;
     d_diag_off_ = nullptr;
+    d_res_jobs_ = nullptr;
+    d_res_parts_ = nullptr;
     pool_ = nullptr;
     pool_alt_ = nullptr;
     d_blocks_ = nullptr;
@@ -215,7 +218,7 @@ int Batch::upload()
     kinds_.clear();
     for (Circ& c : circs_) {
         c.plan.reset();
-        c.solo = c.herm = false;
+        c.solo = c.herm = c.resident = false;
         c.solo_launches = 0;
     }
     std::vector<FusedBlock> blocks;
@@ -224,6 +227,7 @@ int Batch::upload()
     uint64_t off = 0;
     bool any_perm = false;
     std::vector<uint8_t> kinds;
+    std::vector<ResidentPart> parts;
     for (Circ& c : circs_) {
         c.blk_off = blocks.size();
         c.bytes = 0;
@@ -260,6 +264,23 @@ int Batch::upload()
             continue;
         }
         const double sweep = 32.0 * (double)(1ull << (2 * c.n));
+        if (!sweeps_asked_ && resident_wanted(c.gates, c.n, 4)) {
+            FusedPlan* p = nullptr;
+            PlanInfo pi;
+            int rc = build_fused_plan(c.gates, c.n, 4, nullptr, 0, true, &p, &pi, false, false, false,
+                                      true);
+            if (rc) return rc;
+            std::unique_ptr<FusedPlan> hold(p);
+            if (p && p->resident()) {
+                c.resident = true;
+                c.n_blocks = c.n > kResidentColumnQubits ? 3 : 2;  // its launches
+                c.bytes = p->bytes(c.n);
+                c.job = p->resident_job();
+                c.parts_off = parts.size();
+                parts.insert(parts.end(), p->resident_parts().begin(), p->resident_parts().end());
+                continue;
+            }
+        }
         if (hermitian_ && c.n >= kBatchHermQubits) {
             // Hermitian sweeps and relabellings, planned as the single-circuit
             // engine plans with Hermitian sweeps from 8 qubits
@@ -384,6 +405,11 @@ int Batch::upload()
     for (size_t i = 0; i < circs_.size(); i++) {
         Circ& c = circs_[i];
         if (c.solo) continue;  // final_alt set with its plan
+        if (c.resident) {  // in place
+            c.final_alt = false;
+            planes(c, false, c.job.re, c.job.im);
+            continue;
+        }
         bool alt = false;
         for (size_t b = 0; b < c.n_blocks; b++) {
             alt_before[i].push_back(alt ? 1 : 0);
@@ -420,7 +446,8 @@ int Batch::upload()
     // count, tile width).  A group runs all its steps before the next starts,
     // so with a budget below the Infinity Cache its rho stay in the cache
     // from one step to the next.  Returns the number of groups.
-    auto build = [&](uint64_t budget, std::vector<BatchEntry>& ents, std::vector<Launch>& lst) {
+    auto build = [&](uint64_t budget, std::vector<BatchEntry>& ents,
+                     std::vector<ResidentJob>& jobs, std::vector<Launch>& lst) {
         size_t n_groups = 0;
         for (int w = 0; w < (int)waves(); w++) {
             std::vector<int> ids;
@@ -449,13 +476,34 @@ int Batch::upload()
                     // per (qubit count, step kind, tile width)
                     std::map<std::tuple<int, int, int>, std::vector<int>> by;
                     for (int i : grp)
-                        if (s < circs_[i].n_blocks) {
+                        if (s < circs_[i].n_blocks && circs_[i].resident) {
+                            const bool flip = circs_[i].n_blocks == 3;
+                            const int kind = s == 0 || s == 2 ? SK_ROWS : flip ? SK_FLIP : SK_COLUMNS;
+                            by[{resident_log_entries(circs_[i].n), kind, 0}].push_back(i);
+                        } else if (s < circs_[i].n_blocks) {
                             const size_t b = circs_[i].blk_off + s;
                             const int kind = kinds_[b];
                             const int m = kind == SK_INORDER ? (int)blocks[b].m : 8;
                             by[{circs_[i].n, kind, m}].push_back(i);
                         }
-                    for (const auto& kv : by) {
+                    for (auto& kv : by) {
+                        const int kind = std::get<1>(kv.first), L = std::get<0>(kv.first);
+                        if (kind == SK_FLIP) {
+                            for (int i : kv.second) {
+                                lst.push_back(Launch{L, 0, 1, jobs.size(), w, kind});
+                                jobs.push_back(circs_[i].job);
+                            }
+                            continue;
+                        }
+                        if (kind == SK_ROWS || kind == SK_COLUMNS) {
+                            // the longest first, so that the last to end are short
+                            std::stable_sort(kv.second.begin(), kv.second.end(), [&](int a, int b) {
+                                return circs_[a].job.blocks > circs_[b].job.blocks;
+                            });
+                            lst.push_back(Launch{L, 0, (int)kv.second.size(), jobs.size(), w, kind});
+                            for (int i : kv.second) jobs.push_back(circs_[i].job);
+                            continue;
+                        }
                         lst.push_back(Launch{std::get<0>(kv.first), std::get<2>(kv.first),
                                              (int)kv.second.size(), ents.size(), w,
                                              std::get<1>(kv.first)});
@@ -474,7 +522,20 @@ int Batch::upload()
         }
     }
     std::vector<BatchEntry> entries;
-    groups_ = (uint32_t)build(group_bytes_, entries, launches_);
+    if (!parts.empty()) {
+        BTRY(hipMalloc(&d_res_parts_, parts.size() * sizeof(ResidentPart)));
+        BTRY(hipMemcpy(d_res_parts_, parts.data(), parts.size() * sizeof(ResidentPart),
+                       hipMemcpyHostToDevice));
+        for (Circ& c : circs_)
+            if (c.resident) c.job.parts = d_res_parts_ + c.parts_off;
+    }
+    res_jobs_.clear();
+    groups_ = (uint32_t)build(group_bytes_, entries, res_jobs_, launches_);
+    if (!res_jobs_.empty()) {
+        BTRY(hipMalloc(&d_res_jobs_, res_jobs_.size() * sizeof(ResidentJob)));
+        BTRY(hipMemcpy(d_res_jobs_, res_jobs_.data(), res_jobs_.size() * sizeof(ResidentJob),
+                       hipMemcpyHostToDevice));
+    }
     if (!entries.empty()) BTRY(hipMalloc(&d_entries_, entries.size() * sizeof(BatchEntry)));
 
     std::vector<EnergyJob> jobs;
@@ -553,7 +614,7 @@ int Batch::autotune(std::vector<FusedBlock>& blocks)
 {
     std::map<int, std::vector<int>> by_n;  // circuits of in-order blocks by qubit count
     for (int i = 0; i < (int)circs_.size(); i++)
-        if (circs_[i].n_blocks > 0 && !circs_[i].herm) by_n[circs_[i].n].push_back(i);
+        if (circs_[i].n_blocks > 0 && !circs_[i].herm && !circs_[i].resident) by_n[circs_[i].n].push_back(i);
     if (by_n.empty()) return DMX_OK;
     BTRY(hipMemsetAsync(pool_, 0, pool_doubles_ * sizeof(double), stream_));
     size_t most = 0;
@@ -602,7 +663,7 @@ int Batch::autotune(std::vector<FusedBlock>& blocks)
     (void)hipFree(d_tmp);
     if (rc) return rc;
     for (const Circ& c : circs_)
-        if (!c.herm)
+        if (!c.herm && !c.resident)
             for (size_t b = 0; b < c.n_blocks; b++)
                 blocks[c.blk_off + b].m = (uint32_t)tile_bits_[c.n];
     return DMX_OK;
@@ -622,7 +683,11 @@ int Batch::autotune_groups(const LaunchBuilder& build)
     std::vector<Launch> lsts[kCands];
     size_t most = 1;
     for (int c = 0; c < kCands; c++) {
-        build(cands[c], ents[c], lsts[c]);
+        std::vector<ResidentJob> none;  // their rho are not read again: nothing to time
+        build(cands[c], ents[c], none, lsts[c]);
+        lsts[c].erase(std::remove_if(lsts[c].begin(), lsts[c].end(),
+                                     [](const Launch& l) { return l.kind >= SK_ROWS; }),
+                      lsts[c].end());
         most = std::max(most, ents[c].size());
     }
     BTRY(hipMemsetAsync(pool_, 0, pool_doubles_ * sizeof(double), stream_));
@@ -662,6 +727,13 @@ int Batch::autotune_groups(const LaunchBuilder& build)
 
 hipError_t Batch::launch(const Launch& l, const BatchEntry* d_entries)
 {
+    if (l.kind == SK_FLIP) {
+        const ResidentJob& j = res_jobs_[l.entry_off];
+        return launch_conj_transpose(j.re, j.im, j.n, stream_);
+    }
+    if (l.kind == SK_ROWS || l.kind == SK_COLUMNS)
+        return launch_resident_batch(d_res_jobs_ + l.entry_off, l.count, l.n, l.kind == SK_COLUMNS,
+                                     stream_);
     const BatchEntry* e = d_entries + l.entry_off;
     switch (l.kind) {
     case SK_HERM: return launch_fused4_herm_batch(e, l.count, l.n, herm_batch_blocks(l.n), stream_);
@@ -677,6 +749,7 @@ int Batch::set_hermitian(bool on)
         return DMX_ESTATE;
     }
     hermitian_ = on;
+    sweeps_asked_ = true;
     return DMX_OK;
 }
 

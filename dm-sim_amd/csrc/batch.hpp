@@ -97,6 +97,9 @@ public:
     // few items to fill the GPU.
     int set_hermitian(bool on);
     static constexpr int kBatchHermQubits = 10;
+    // Until set_hermitian asks for one form of sweep or the other, the batched
+    // circuits run on resident rows (resident.hpp), every circuit of a wave's
+    // group and width in two launches (and conjugate transposes from 10 qubits).
     // Workgroups of one batched Hermitian launch in all (shared among its
     // circuits), so that each takes several upper-tile items in turn and its
     // next item's loads overlap the transform.  256 hardware-efficient
@@ -127,6 +130,9 @@ private:
         std::vector<Gate> orig;   // as added
         std::vector<Gate> gates;  // C4X expanded (batched blocks have at most four qubits)
         bool solo = false;        // runs on its own (kSoloQubits and up)
+        bool resident = false;    // its blocks run on resident rows
+        size_t parts_off = 0;     // its records
+        ResidentJob job = {};
         bool herm = false;        // its batched steps are Hermitian sweeps and relabellings
         double bytes = 0;         // algorithmic bytes of its steps
         std::unique_ptr<FusedPlan> plan;  // its plan then
@@ -139,18 +145,26 @@ private:
         int wave = 0;
         uint64_t diag_off = 0;  // its diagonal in the kept diagonals (several waves)
     };
-    enum StepKind : uint8_t { SK_INORDER = 0, SK_HERM = 1, SK_RELABEL = 2 };
+    enum StepKind : uint8_t {
+        SK_INORDER = 0,
+        SK_HERM = 1,
+        SK_RELABEL = 2,
+        SK_ROWS = 3,  // resident rows, the column index
+        SK_COLUMNS = 4,  // and the row index (up to kResidentColumnQubits)
+        SK_FLIP = 5  // one circuit's conjugate transpose, between two SK_ROWS
+    };
     struct Launch {
         int n;
         int m;
         int count;
-        size_t entry_off;
+        size_t entry_off;  // into the entries, or (resident) the jobs
         int wave;
         int kind;  // StepKind
     };
     hipError_t launch(const Launch& l, const BatchEntry* d_entries);
     using LaunchBuilder =
-        std::function<size_t(uint64_t, std::vector<BatchEntry>&, std::vector<Launch>&)>;
+        std::function<size_t(uint64_t, std::vector<BatchEntry>&, std::vector<ResidentJob>&,
+                             std::vector<Launch>&)>;
     int enqueue();  // the whole run on stream_ (captured or eager)
     int autotune_groups(const LaunchBuilder& build);
     int autotune(std::vector<FusedBlock>& blocks);
@@ -160,6 +174,10 @@ private:
     std::vector<Launch> launches_;
     CostModel* model_ = nullptr;
     bool hermitian_ = true;
+    bool sweeps_asked_ = false;  // set_hermitian was called
+    std::vector<ResidentJob> res_jobs_;
+    ResidentJob* d_res_jobs_ = nullptr;
+    ResidentPart* d_res_parts_ = nullptr;
     std::vector<uint8_t> kinds_;  // StepKind of every batched step (parallel to the blocks)
     LaunchProfiler quiet_;  // disabled: the solo plans' executor times nothing
     bool uploaded_ = false;

@@ -147,6 +147,12 @@ struct Plan : FusedPlan {
 
     bool resident() const override { return !rparts.empty(); }
 
+    const std::vector<ResidentPart>& resident_parts() const override { return rparts; }
+
+    ResidentJob resident_job() const override
+    {
+        return ResidentJob{nullptr, nullptr, d_rparts, (int)steps.size(), n, rend};
+    }
 
     bool flips() const override { return !rparts.empty() && n > kResidentColumnQubits; }
 
@@ -291,9 +297,10 @@ struct Plan : FusedPlan {
                 la++;
             };
             auto pass = [&](bool slow) {
-                launch(KC_RESIDENT, [&] {
-                    return launch_resident(re, im, d_rparts, (int)steps.size(), rend, nq, slow, stream);
-                });
+                ResidentJob job = resident_job();
+                job.re = re;
+                job.im = im;
+                launch(KC_RESIDENT, [&] { return launch_resident(job, slow, stream); });
             };
             pass(false);
             if (flips()) launch(KC_TRANSPOSE, [&] { return launch_conj_transpose(re, im, nq, stream); });

@@ -11,6 +11,7 @@
 #include "fused.hpp"
 #include "group.hpp"
 #include "prof.hpp"
+#include "resident.hpp"
 
 namespace dmx {
 
@@ -68,6 +69,9 @@ struct FusedPlan {
     virtual bool staged() const = 0;
     // Whether every block runs on resident rows (resident.hpp) instead of in sweeps.
     virtual bool resident() const = 0;
+    // Their records on the host (d_parts not set), for batched launches.
+    virtual const std::vector<ResidentPart>& resident_parts() const = 0;
+    virtual ResidentJob resident_job() const = 0;
     // Whether execute leaves rho in the other orientation (conj-transposed).
     virtual bool flips() const = 0;
     // Whether execute needs a second pair of planes (blocks with a trailing

@@ -30,10 +30,13 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c)
 // n <= LOGE; a chunk is 2^LOGE entries, 2^(LOGE - 8) tiles, dealt to the waves
 // in runs.  SLOW: rows and columns of rho exchanged, and conjugated values.
 template <int LOGE, int WAVES, bool SLOW>
-__global__ void __launch_bounds__(64 * WAVES, 4)
-    k_resident(double* __restrict__ re, double* __restrict__ im, const double2* __restrict__ parts,
-               int blocks, ResidentEnd end, int n)
+__device__ __forceinline__ void resident_pass(const ResidentJob& job)
 {
+    double* const re = job.re;
+    double* const im = job.im;
+    const double2* const parts = reinterpret_cast<const double2*>(job.parts);
+    const int blocks = job.blocks, n = job.n;
+    const ResidentEnd& end = job.end;
     constexpr int kThreads = 64 * WAVES;
     constexpr int kPer = (1 << (LOGE - 8)) / WAVES;  // tiles of a wave
     __shared__ double2 s[1 << LOGE];
@@ -107,24 +110,25 @@ __global__ void __launch_bounds__(64 * WAVES, 4)
         for (int u = 0; u < kPer; u++)
 #pragma unroll
             for (int c = 0; c < 4; c++) v[u][c] = s[x[u][c]];
-        // three real products, the additions left to the accumulators: with
-        // K = Ur (Xr + Xi), re = K - (Ur + Ui) Xi and im = K + (Ui - Ur) Xr
-        d4 yr[kPer], yi[kPer];
+        // three real products, p1 = Ur Xr (in yr), p2 = Ui Xi and, in yi, (Ur + Ui) (Xr + Xi)
+        // (as four chained by their accumulators 601 gates at n = 11 take 700 us
+        // a pass for 651, and the results are a little further off)
+        d4 yr[kPer], yi[kPer], p2[kPer];
 #pragma unroll
-        for (int u = 0; u < kPer; u++) yr[u] = d4{0, 0, 0, 0};
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int u = 0; u < kPer; u++) yr[u] = mfma(ur[c], v[u][c].x + v[u][c].y, yr[u]);
-#pragma unroll
-        for (int u = 0; u < kPer; u++) yi[u] = yr[u];
+        for (int u = 0; u < kPer; u++) yr[u] = yi[u] = p2[u] = d4{0, 0, 0, 0};
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int u = 0; u < kPer; u++) {
-                yr[u] = mfma(-ur[c] - ui[c], v[u][c].y, yr[u]);
-                yi[u] = mfma(ui[c] - ur[c], v[u][c].x, yi[u]);
+                yr[u] = mfma(ur[c], v[u][c].x, yr[u]);
+                p2[u] = mfma(ui[c], v[u][c].y, p2[u]);
+                yi[u] = mfma(ur[c] + ui[c], v[u][c].x + v[u][c].y, yi[u]);
             }
+#pragma unroll
+        for (int u = 0; u < kPer; u++) {
+            yi[u] = yi[u] - yr[u] - p2[u];
+            yr[u] = yr[u] - p2[u];
+        }
 #pragma unroll
         for (int u = 0; u < kPer; u++)
 #pragma unroll
@@ -160,25 +164,52 @@ __global__ void __launch_bounds__(64 * WAVES, 4)
     }
 }
 
-hipError_t launch_resident(double* re, double* im, const ResidentPart* d_parts, int blocks,
-                           const ResidentEnd& end, int n, bool slow, hipStream_t stream)
+template <int LOGE, int WAVES, bool SLOW>
+__global__ void __launch_bounds__(64 * WAVES, 4) k_resident(const ResidentJob job)
 {
-    if (n < 4 || n > (slow ? kResidentColumnQubits : kResidentMaxQubits) || blocks < 1)
+    resident_pass<LOGE, WAVES, SLOW>(job);
+}
+
+template <int LOGE, int WAVES, bool SLOW>
+__global__ void __launch_bounds__(64 * WAVES, 4) k_resident_batch(const ResidentJob* __restrict__ jobs)
+{
+    const ResidentJob& job = jobs[blockIdx.y];
+    if (blockIdx.x >= 1u << (2 * job.n - LOGE)) return;  // a narrower circuit's
+    resident_pass<LOGE, WAVES, SLOW>(job);
+}
+
+hipError_t launch_resident(const ResidentJob& job, bool slow, hipStream_t stream)
+{
+    const int n = job.n;
+    if (n < 4 || n > (slow ? kResidentColumnQubits : kResidentMaxQubits) || job.blocks < 1)
         return hipErrorInvalidValue;
-    const unsigned grid = 1u << (2 * n - resident_log_entries(n));
-    const double2* p = reinterpret_cast<const double2*>(d_parts);
-    if (slow) {
-        if (n <= 8)
-            k_resident<8, 1, true><<<grid, 64, 0, stream>>>(re, im, p, blocks, end, n);
-        else
-            k_resident<9, 2, true><<<grid, 128, 0, stream>>>(re, im, p, blocks, end, n);
-        return hipGetLastError();
+    const int L = resident_log_entries(n);
+    const unsigned grid = 1u << (2 * n - L);
+    switch (2 * L + (slow ? 1 : 0)) {
+    case 16: k_resident<8, 1, false><<<grid, 64, 0, stream>>>(job); break;
+    case 17: k_resident<8, 1, true><<<grid, 64, 0, stream>>>(job); break;
+    case 18: k_resident<9, 2, false><<<grid, 128, 0, stream>>>(job); break;
+    case 19: k_resident<9, 2, true><<<grid, 128, 0, stream>>>(job); break;
+    case 20: k_resident<10, 4, false><<<grid, 256, 0, stream>>>(job); break;
+    default: k_resident<11, 8, false><<<grid, 512, 0, stream>>>(job); break;
     }
-    switch (n <= 8 ? 8 : n) {
-    case 8: k_resident<8, 1, false><<<grid, 64, 0, stream>>>(re, im, p, blocks, end, n); break;
-    case 9: k_resident<9, 2, false><<<grid, 128, 0, stream>>>(re, im, p, blocks, end, n); break;
-    case 10: k_resident<10, 4, false><<<grid, 256, 0, stream>>>(re, im, p, blocks, end, n); break;
-    default: k_resident<11, 8, false><<<grid, 512, 0, stream>>>(re, im, p, blocks, end, n); break;
+    return hipGetLastError();
+}
+
+hipError_t launch_resident_batch(const ResidentJob* d_jobs, int count, int log_entries, bool slow,
+                                 hipStream_t stream)
+{
+    if (count < 1 || count > 65535 || log_entries < 8 ||
+        log_entries > (slow ? kResidentColumnQubits : kResidentMaxQubits))
+        return hipErrorInvalidValue;
+    const dim3 grid(1u << log_entries, (unsigned)count);  // n = log_entries has the most chunks
+    switch (2 * log_entries + (slow ? 1 : 0)) {
+    case 16: k_resident_batch<8, 1, false><<<grid, 64, 0, stream>>>(d_jobs); break;
+    case 17: k_resident_batch<8, 1, true><<<grid, 64, 0, stream>>>(d_jobs); break;
+    case 18: k_resident_batch<9, 2, false><<<grid, 128, 0, stream>>>(d_jobs); break;
+    case 19: k_resident_batch<9, 2, true><<<grid, 128, 0, stream>>>(d_jobs); break;
+    case 20: k_resident_batch<10, 4, false><<<grid, 256, 0, stream>>>(d_jobs); break;
+    default: k_resident_batch<11, 8, false><<<grid, 512, 0, stream>>>(d_jobs); break;
     }
     return hipGetLastError();
 }

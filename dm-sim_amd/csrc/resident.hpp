@@ -51,9 +51,23 @@ struct ResidentEnd {
 void build_resident(const std::vector<FusedBlock>& blocks, const std::vector<int>& order, int n,
                     std::vector<ResidentPart>& parts, ResidentEnd& end);
 
+// One circuit's rho and its records.
+struct ResidentJob {
+    double* re;
+    double* im;
+    const ResidentPart* parts;
+    int32_t blocks;
+    int32_t n;
+    ResidentEnd end;
+};
+
 // rho <- rho U^T for the product U of all blocks, 4 <= n <= kResidentMaxQubits;
 // slow (n <= kResidentColumnQubits): rho <- conj(U) rho.  In place.
-hipError_t launch_resident(double* re, double* im, const ResidentPart* d_parts, int blocks,
-                           const ResidentEnd& end, int n, bool slow, hipStream_t stream);
+hipError_t launch_resident(const ResidentJob& job, bool slow, hipStream_t stream);
+
+// The same for `count` circuits whose chunks have 2^log_entries entries
+// (resident_log_entries of every job's n, so one launch takes all widths up to 8).
+hipError_t launch_resident_batch(const ResidentJob* d_jobs, int count, int log_entries, bool slow,
+                                 hipStream_t stream);
 
 }  // namespace dmx

@@ -61,3 +61,43 @@ def test_resident_runs_match_plain(n, first):
     s.set_profiling(True)
     s.run()
     assert s.profile()["k_resident"]["calls"] == 2
+
+
+@pytest.mark.gpu
+def test_resident_batch_equals_single_runs():
+    """Batched circuits of uneven width and depth against each circuit's own
+    run (its result in the same orientation), bit for bit, in one wave and, by a pool
+    limit, in several."""
+    import dmsim_amd as dm
+    rng = np.random.default_rng(5)
+    items = []
+    for n in (4, 11, 6, 8, 9, 10, 7, 5, 9, 11):
+        strings, weights = W.random_paulis(n, 4, rng)
+        items.append((W.hea_circuit(n, int(rng.integers(1, 9)), rng), strings, weights))
+    diags = []
+    for limit in (0, 16 << 22):
+        b = dm.Batch()
+        b.set_pool_limit(limit)
+        for circ, strings, weights in items:
+            b.add_circuit(circ, strings, weights)
+        b.upload()
+        b.run()
+        b.run()
+        diags.append([b.get_diag(i) for i in range(len(items))] + [b.energies()])
+        if limit == 0:
+            assert b.stats()["launches"] < 20
+            for cid, (circ, _, _) in enumerate(items):
+                s = dm.Sim(circ.n_qubits)
+                s.set_method(dm.METHOD_FUSED)
+                s.append_table(circ)
+                s.upload()
+                s.run()
+                re, im = s.get_dm()
+                bre, bim = b.get_dm(cid)
+                if circ.n_qubits > 9:  # the batch leaves rho conj-transposed
+                    d = 1 << circ.n_qubits
+                    bre, bim = bre.reshape(d, d).T.ravel(), -bim.reshape(d, d).T.ravel()
+                assert np.array_equal(re, bre) and np.array_equal(im, bim), cid
+        b.close()
+    for x, y in zip(*diags):
+        assert np.array_equal(x, y)
