@@ -1881,17 +1881,27 @@ int choose_executions(const std::vector<Gate>& circuit, int n, BlockPlan& bp, Co
     int rc = model.price(feats, us);
     if (rc) return rc;
     const int m_default = herm ? 4 : default_tile_bits(n);  // herm: the one option, slot 0
+    // A block's width: the one the network prices fastest, but the one most
+    // blocks get unless it is predicted clearly slower (its errors there reach
+    // the difference of neighbouring widths: at n = 10 widths 7 and 8 take 11.6 and
+    // 13.3 us a launch, 17.2 and 13.3 for blocks on high qubits).
+    auto fastest = [&](int b) {
+        const float* t = us.data() + first[b];
+        int m = m_default;
+        for (int i = 0; i < n_m && !herm; i++)
+            if (tile_bits_ok(n, 4 + i, bp.blocks[b].qmask) && t[i] < t[m - 4]) m = 4 + i;
+        return m;
+    };
+    int votes[9] = {}, usual = m_default;
+    for (int b = 0; b < nb && !herm; b++) votes[fastest(b)]++;
+    for (int m = 4; m <= m_hi; m++)
+        if (votes[m] > votes[usual]) usual = m;
     for (int b = 0; b < nb; b++) {
         const float* t = us.data() + first[b];
-        // the width the network prices fastest (one kernel at different
-        // widths: no margin, its errors there are alike)
-        int best_m = m_default;
-        double best = t[m_default - 4];
-        for (int i = 0; i < n_m && !herm; i++)
-            if (tile_bits_ok(n, 4 + i, bp.blocks[b].qmask) && t[i] < best) {
-                best_m = 4 + i;
-                best = t[i];
-            }
+        int best_m = fastest(b);
+        if (tile_bits_ok(n, usual, bp.blocks[b].qmask) && t[best_m - 4] > kMargin * t[usual - 4])
+            best_m = usual;
+        double best = t[best_m - 4];
         if (herm) best_m = 8;
         info.greedy_us += t[m_default - 4];
         bool use_plain = false;
