@@ -327,16 +327,15 @@ def batched(steps, warmup, seed=4, n_circuits=256, trace=False):
             out["launches_per_run"] = st["launches"]
             out["tile_bits"] = {n: b.tile_bits(n) for n in range(6, 12)}
             out["schedule"] = b.schedule()
-            # the batched run's block sweeps: 32 * 4^n bytes each, over the
+            # the batched run's passes over rho: 32 * 4^n bytes each, over the
             # run's device time (which also holds the reset and the energies)
             out["roofline"] = {
                 "bound": "hbm", "achieved": st["sweep_bytes"] / (st["ms"] * 1e-3) / 1e9,
                 "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": st["sweep_bytes"] / (st["ms"] * 1e-3) / 1e9 / HBM_PEAK_GBS,
                 "bytes_per_run": st["sweep_bytes"], "device_ms_per_run": st["ms"],
-                "note": "one circuit's rho (<= 67 MB at 11 qubits) fits the 256 MB Infinity "
-                        "Cache, but a launch sweeps all circuits of one width (up to 3.3 GB): "
-                        "the 10- and 11-qubit steps stream from HBM",
+                "note": "rho moves through memory two or three times a run, its rows held on "
+                        "chip for all blocks between: the run's time is FP64 matrix work",
             }
         b.close()
     if trace:

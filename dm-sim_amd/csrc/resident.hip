@@ -10,6 +10,16 @@
 // bits: a lane reads and writes the same four places, so a block takes one barrier
 // (none where a wave holds the row, up to 8 qubits).  Index permutations between
 // blocks (X, CX, SWAP) only change the places that later records name.
+//
+// Bound: up to 9 qubits one wave's chain of LDS reads, 12 MFMAs and LDS writes (0.64
+// us a block and pass at n = 8, where 256 waves have a SIMD each); from 10 the FP64
+// matrix cores, busy 64 % of the time at n = 11 with eight waves of a tile each (9.1
+// us a block and pass for 6.2 at 65 TFLOP/s; LDS 19 % of the time, 15 % of that
+// bank conflicts).  There four waves of two tiles, one after the other, leave
+// registers for five workgroups a CU instead of two: 601 gates 665 -> 638 us a pass,
+// 96 circuits of 6 to 11 qubits 16.4 -> 14.9 ms.
+// Against one launch per block: 90 blocks at n = 8 586 -> 117 us a run, 30 at n = 11
+// 1305 -> 560.
 #include <hip/hip_runtime.h>
 
 #include "resident.hpp"
@@ -87,52 +97,39 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
         const uint32_t w2 = (uint32_t)__double2loint(next[4].y);
         const uint32_t c0 = w0 >> 16, c1 = w1 & 0xFFFFu;
         const uint32_t t[3] = {w1 >> 16, w2 & 0xFFFFu, w2 >> 16};
-        uint32_t x[kPer][4];
-#pragma unroll
-        for (int u = 0; u < kPer; u++) {
-            const uint32_t tile = wave * kPer + u;
-            uint32_t base = w0 & 0xFFFFu;
-#pragma unroll
-            for (int i = 0; i < LOGE - 8; i++) base ^= (tile >> i) & 1u ? t[i] : 0u;
-            x[u][0] = base;
-            x[u][1] = base ^ c0;
-            x[u][2] = base ^ c1;
-            x[u][3] = base ^ c0 ^ c1;
-        }
         src += 64 * kResidentParts;
         __syncthreads();
         if (b + 1 < blocks) {
 #pragma unroll
             for (int i = 0; i < kResidentParts; i++) next[i] = src[64 * i];
         }
-        double2 v[kPer][4];
-#pragma unroll
-        for (int u = 0; u < kPer; u++)
-#pragma unroll
-            for (int c = 0; c < 4; c++) v[u][c] = s[x[u][c]];
-        // three real products, p1 = Ur Xr (in yr), p2 = Ui Xi and, in yi, (Ur + Ui) (Xr + Xi)
-        // (as four chained by their accumulators 601 gates at n = 11 take 700 us
-        // a pass for 651, and the results are a little further off)
-        d4 yr[kPer], yi[kPer], p2[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; u++) yr[u] = yi[u] = p2[u] = d4{0, 0, 0, 0};
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int u = 0; u < kPer; u++) {
-                yr[u] = mfma(ur[c], v[u][c].x, yr[u]);
-                p2[u] = mfma(ui[c], v[u][c].y, p2[u]);
-                yi[u] = mfma(ur[c] + ui[c], v[u][c].x + v[u][c].y, yi[u]);
-            }
-#pragma unroll
+#pragma unroll 1
         for (int u = 0; u < kPer; u++) {
-            yi[u] = yi[u] - yr[u] - p2[u];
-            yr[u] = yr[u] - p2[u];
+            const uint32_t tile = wave * kPer + u;
+            uint32_t x[4] = {w0 & 0xFFFFu};
+#pragma unroll
+            for (int i = 0; i < LOGE - 8; i++) x[0] ^= (tile >> i) & 1u ? t[i] : 0u;
+            x[1] = x[0] ^ c0;
+            x[2] = x[0] ^ c1;
+            x[3] = x[1] ^ c1;
+            double2 v[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = s[x[c]];
+            // three real products, p1 = Ur Xr (in yr), p2 = Ui Xi and, in yi, (Ur + Ui) (Xr +
+            // Xi) (as four chained by their accumulators 601 gates at n = 11 take
+            // 700 us a pass for 651, and the results are a little further off)
+            d4 yr = {0, 0, 0, 0}, yi = yr, p2 = yr;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                yr = mfma(ur[c], v[c].x, yr);
+                p2 = mfma(ui[c], v[c].y, p2);
+                yi = mfma(ur[c] + ui[c], v[c].x + v[c].y, yi);
+            }
+            yi = yi - yr - p2;
+            yr = yr - p2;
+#pragma unroll
+            for (int r = 0; r < 4; r++) s[x[r]] = make_double2(yr[r], yi[r]);
         }
-#pragma unroll
-        for (int u = 0; u < kPer; u++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) s[x[u][r]] = make_double2(yr[u][r], yi[u][r]);
     }
     __syncthreads();
 
@@ -165,13 +162,13 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
 }
 
 template <int LOGE, int WAVES, bool SLOW>
-__global__ void __launch_bounds__(64 * WAVES, 4) k_resident(const ResidentJob job)
+__global__ void __launch_bounds__(64 * WAVES, 5) k_resident(const ResidentJob job)
 {
     resident_pass<LOGE, WAVES, SLOW>(job);
 }
 
 template <int LOGE, int WAVES, bool SLOW>
-__global__ void __launch_bounds__(64 * WAVES, 4) k_resident_batch(const ResidentJob* __restrict__ jobs)
+__global__ void __launch_bounds__(64 * WAVES, 5) k_resident_batch(const ResidentJob* __restrict__ jobs)
 {
     const ResidentJob& job = jobs[blockIdx.y];
     if (blockIdx.x >= 1u << (2 * job.n - LOGE)) return;  // a narrower circuit's
@@ -191,7 +188,7 @@ hipError_t launch_resident(const ResidentJob& job, bool slow, hipStream_t stream
     case 18: k_resident<9, 2, false><<<grid, 128, 0, stream>>>(job); break;
     case 19: k_resident<9, 2, true><<<grid, 128, 0, stream>>>(job); break;
     case 20: k_resident<10, 4, false><<<grid, 256, 0, stream>>>(job); break;
-    default: k_resident<11, 8, false><<<grid, 512, 0, stream>>>(job); break;
+    default: k_resident<11, 4, false><<<grid, 256, 0, stream>>>(job); break;
     }
     return hipGetLastError();
 }
@@ -209,7 +206,7 @@ hipError_t launch_resident_batch(const ResidentJob* d_jobs, int count, int log_e
     case 18: k_resident_batch<9, 2, false><<<grid, 128, 0, stream>>>(d_jobs); break;
     case 19: k_resident_batch<9, 2, true><<<grid, 128, 0, stream>>>(d_jobs); break;
     case 20: k_resident_batch<10, 4, false><<<grid, 256, 0, stream>>>(d_jobs); break;
-    default: k_resident_batch<11, 8, false><<<grid, 512, 0, stream>>>(d_jobs); break;
+    default: k_resident_batch<11, 4, false><<<grid, 256, 0, stream>>>(d_jobs); break;
     }
     return hipGetLastError();
 }
