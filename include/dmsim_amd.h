@@ -169,7 +169,11 @@ int dmx_set_fusion_permute(dmx_sim* sim, uint32_t on);
  * conjugate transpose; rho's index bits are relabelled between blocks and
  * restored at the end of the run).  mode 0 = off, 1 = from 12 qubits
  * (default), 2 = from 8 qubits.  Out of place: uses the second pair of
- * planes.  Used from the next dmx_upload. */
+ * planes.  Used from the next dmx_upload.
+ *
+ * With mode 1, permuting blocks on, no fixed tile width and blocks of at most
+ * four qubits, unitary circuits of 4 to 11 qubits make no sweeps: all blocks run
+ * in two launches that hold whole rows of rho on chip. */
 int dmx_set_fusion_hermitian(dmx_sim* sim, uint32_t mode);
 
 /* Extension: the greedy plan's tile width measured (on = 1, default): without
@@ -177,7 +181,8 @@ int dmx_set_fusion_hermitian(dmx_sim* sim, uint32_t mode);
  * the plan's block sweeps at every tile width on scratch planes (rho is not
  * touched) and runs every block at the fastest width where it is admissible;
  * off = 0 keeps the default width min(8, n).  dmx_tuned_tile_bits reports the
- * width the last upload chose (0: none timed). */
+ * width the last upload chose (0: none timed, as where blocks run on rows held on
+ * chip and no sweep has a width). */
 int dmx_set_fusion_autotune(dmx_sim* sim, uint32_t on);
 int dmx_tuned_tile_bits(const dmx_sim* sim, uint32_t* m);
 
@@ -310,7 +315,8 @@ int dmx_set_tile_bits(dmx_sim* sim, uint32_t m);
  * fused (a five-qubit block the model splits counts as its four-qubit
  * sub-blocks instead), the model's predicted device time of the blocks'
  * launches and its prediction for the same blocks fused at the default width
- * (microseconds; 0 without a model), and tiles[5] = fused four-qubit blocks
+ * (microseconds; 0 without a model; both as block sweeps, also where the blocks
+ * run on rows held on chip), and tiles[5] = fused four-qubit blocks
  * per tile width m = 4..8 (may be NULL). */
 int dmx_plan_info(const dmx_sim* sim, uint32_t* fused_blocks, uint32_t* plain_blocks,
                   uint32_t* fused5_blocks, double* predicted_us, double* greedy_us,
