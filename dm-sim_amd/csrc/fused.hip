@@ -97,12 +97,12 @@ __device__ __forceinline__ uint64_t deposit(uint64_t v, uint64_t mask)
 // stage's matrix is loaded once for the wave's tiles.  col(tb, b): LDS column of
 // local column b of tile tb; at(a, x): LDS place of row a, column x.
 // A superoperator stage is Y = S X with X's rows the 16 (row, column) values of
-// bits u, v and X's columns the 16 of the other two: 12 MFMAs (one complex
-// product) against the 24 of a unitary stage, and a lane reads and writes the
-// same four places.  Bound like the sweep around it by memory up to about four
-// stages a block (4 stages of 12 MFMAs take as long as a Hermitian sweep's
-// traffic at 60 TFLOP/s), by the FP64 MFMA rate above: at n = 14, 38 noisy
-// sweeps take 1.51 ms each where 32 unitary ones take 0.98.
+// bits u, v and X's columns the 16 of the other two: 16 MFMAs (one complex
+// product as four real ones: the errors of a noisy 8-qubit circuit are those of
+// single channels, 1.9e-15 over three inputs, where three products gave 2.3e-15 in
+// the same 222 us a pass) against the 24 of a unitary stage, and a lane reads and
+// writes the same four places.  Bound like the sweep around it by memory up to about three
+// stages a block, by the FP64 MFMA rate above.
 template <int NTILES, class On, class Col, class At>
 __device__ __forceinline__ void run_stages(const FusedStage* __restrict__ stages, uint32_t count,
                                            int wave, int lane, const On& on, const Col& col,
@@ -163,17 +163,16 @@ __device__ __forceinline__ void run_stages(const FusedStage* __restrict__ stages
         for (int tb = wave; tb < NTILES; tb += 4) {
             if (!on(tb)) continue;
             const int x0 = col(tb, b);
-            d4 p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0}, p3 = {0, 0, 0, 0};
+            d4 yr = {0, 0, 0, 0}, yi = yr;  // four real products
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const int x = at(row[c], x0);
                 const double tr = s_re[x], ti = s_im[x];
-                p1 = mfma(ur[c], tr, p1);
-                p2 = mfma(ui[c], ti, p2);
-                p3 = mfma(ur[c] + ui[c], tr + ti, p3);
+                yr = mfma(ur[c], tr, yr);
+                yi = mfma(ur[c], ti, yi);
+                yr = mfma(-ui[c], ti, yr);
+                yi = mfma(ui[c], tr, yi);
             }
-            const d4 yr = p1 - p2;
-            const d4 yi = p3 - p1 - p2;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int x = at(row[r], x0);
