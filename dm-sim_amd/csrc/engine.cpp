@@ -293,19 +293,58 @@ uint64_t Engine::device_bytes() const
     return b;
 }
 
+namespace {
+
+// A segment's time either way, in passes that read and write rho once (all launches
+// stream rho: 72 us at 12 qubits, 430 at 13, 1800 at 14; below 10 qubits a launch is
+// about 3 us whatever it moves).  A sweep of a dense pair or 4 x 4 primitive is one
+// pass; one of a diagonal kind or CX, which touches half of the entries, measures
+// 0.6 to 0.8.  On rows a segment of any length takes two passes, which at 14 qubits,
+// one row to a CU, measure 1.75 each, with a conjugate transpose between them, and
+// one before them if rho is held transposed.  One H at 13 qubits 0.87 ms as sweeps and 1.32
+// on rows, at 14 3.6 and 8.1; two H 1.7 and 1.3, 7.0 and 8.1.
+double sweep_passes(const PrimOp& p)
+{
+    const int c = prim_class(p);
+    return c == KC_CX || c == KC_PAIR_POS1 ? 0.7 : 1.0;
+}
+double row_passes(int n, bool transposed) { return (n < 14 ? 3.0 : 4.5) + (transposed ? 1.0 : 0.0); }
+
+}  // namespace
+
 int Engine::ensure_rows()
 {
     if (!row_first_.empty() || prims_.empty()) return DMX_OK;
     std::vector<RowOp> prog;
     std::vector<size_t> first;
+    std::vector<double> sweeps;  // passes of each segment as sweeps
     size_t s0 = 0;
     while (s0 < prims_.size()) {
         size_t s1 = s0;
-        while (s1 < prims_.size() && prims_[s1].kind != PK_SUP) s1++;
-        if (s1 > s0) first.push_back(build_row_program(prims_, s0, s1, n_, prog));
+        double cost = 0;
+        while (s1 < prims_.size() && prims_[s1].kind != PK_SUP) cost += 2 * sweep_passes(prims_[s1++]);
+        if (s1 > s0) {
+            first.push_back(build_row_program(prims_, s0, s1, n_, prog));
+            sweeps.push_back(cost);
+        }
         s0 = s1 + 2;
     }
     if (first.empty()) return DMX_OK;  // channels only
+    // Sweeps leave rho in the other orientation, rows in the stored one: the cheapest
+    // way through all segments from each orientation, from the last one back.
+    std::vector<uint8_t> on_rows(first.size(), 0);
+    double rest[2] = {0.0, 0.0};
+    for (size_t s = first.size(); s-- > 0;) {
+        double best[2];
+        for (int o = 0; o < 2; o++) {
+            const double as_sweeps = sweeps[s] + rest[1 - o];
+            const double as_rows = row_passes(n_, o == 1) + rest[0];
+            if (as_rows < as_sweeps) on_rows[s] |= (uint8_t)(1u << o);
+            best[o] = std::min(as_rows, as_sweeps);
+        }
+        rest[0] = best[0];
+        rest[1] = best[1];
+    }
     if (prog.size() > d_rows_cap_) {
         if (d_rows_) HIPTRY(hipFree(d_rows_));
         d_rows_ = nullptr;
@@ -317,6 +356,7 @@ int Engine::ensure_rows()
                           stream_));
     HIPTRY(hipStreamSynchronize(stream_));  // the source ends with this call
     row_first_ = std::move(first);
+    on_rows_ = std::move(on_rows);
     return DMX_OK;
 }
 
@@ -351,18 +391,16 @@ int Engine::run_plain(bool per_launch)
     // index passes (the reference's forward and backward pass); a channel then
     // acts once on both indices, in the record for the current orientation.
     int s0 = 0;
-    size_t segment = 0;
-    while (s0 < n_ops) {
+    for (size_t segment = 0; s0 < n_ops;) {
         int s1 = s0;
         while (s1 < n_ops && prims_[s1].kind != PK_SUP) s1++;
-        if (s1 > s0 && rows) {
+        if (s1 > s0 && rows && ((on_rows_[segment] >> (transposed_ ? 1 : 0)) & 1)) {
             // the reference's order: columns, conjugate transpose, columns
             if (transposed_) HIPTRY(transpose());
             transposed_ = false;
             HIPTRY(row_pass(segment));
             HIPTRY(transpose());
             HIPTRY(row_pass(segment));
-            segment++;
             last_sweeps_ += 2u * (uint32_t)(s1 - s0);
         } else if (s1 > s0) {
             // reference orientation: fast index first; transposed: slow first
@@ -380,6 +418,7 @@ int Engine::run_plain(bool per_launch)
             last_sweeps_ += 2u * (uint32_t)(s1 - s0);
             transposed_ = !transposed_;
         }
+        if (s1 > s0) segment++;
         if (s1 < n_ops) {  // channel: records s1 (stored orientation), s1 + 1 (transposed)
             const int pick = s1 + (transposed_ ? 1 : 0);
             prof_.begin(KC_QUAD, prim_bytes(prims_[pick], n_));

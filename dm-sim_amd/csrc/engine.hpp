@@ -115,6 +115,8 @@ private:
     RowOp* d_rows_ = nullptr;  // every segment's program (rows.hpp)
     size_t d_rows_cap_ = 0;
     std::vector<size_t> row_first_;  // first record of each; empty: not built
+    std::vector<uint8_t> on_rows_;   // per segment, bit o: from orientation o (1: transposed) it
+                                     // runs on resident rows, else as its primitives' sweeps
     hipStream_t stream_ = nullptr;
     hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
 

@@ -1,0 +1,62 @@
+"""Short circuits and short stretches of gates between channels: each runs the
+cheaper of its forms, with the same results."""
+import numpy as np
+import pytest
+
+import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 6, 9, 10, 11, 13, 14])
+def test_plain_segments_equal_one_launch_per_primitive(n):
+    """The plain method on segments of one to twelve gates between channels, some on
+    resident rows and some as sweeps, from both orientations, against one launch
+    per primitive bit for bit."""
+    import dmsim_amd as dm
+    rng = np.random.default_rng(40 + n)
+    names = [g for g in W.OP_NAMES if W.ARITY[g] <= min(n, 3)]
+    sims = [dm.Sim(n) for _ in range(4)]
+    for i, size in enumerate((1, 12, 1, 2, 1, 1, 12, 12, 3, 1)):
+        t = W.random_mixed(n, size, 900 + 10 * n + i, gate_set=names)
+        q = int(rng.integers(n))
+        for s in sims:
+            s.append_table(t)
+            s.append_kraus(q, dm.amplitude_damping(0.07))
+    idx = rng.integers(0, 4 ** n, size=4096, dtype=np.uint64)
+    one, rows = dm.METHOD_PLAIN_LAUNCH, dm.METHOD_PLAIN
+    for s, methods in zip(sims, ((rows, rows), (one, one), (one, rows), (rows, one))):
+        s.upload()
+        for m in methods:
+            s.set_method(m)
+            s.run()
+    sims[0].set_profiling(True)
+    sims[0].run()
+    calls = sims[0].profile()
+    assert "k_rows" in calls and any(c.startswith("k_sweep") for c in calls)
+    sims[1].run()
+    want = sims[1].get_entries(idx), sims[1].get_diag()
+    assert np.array_equal(sims[0].get_entries(idx), want[0])
+    assert np.array_equal(sims[0].get_diag(), want[1])
+    for s in sims[2:]:
+        s.run()  # the third run of each, in its last method
+        assert np.array_equal(s.get_entries(idx), want[0])
+        assert np.array_equal(s.get_diag(), want[1])
+
+
+@pytest.mark.parametrize("n", [2, 9, 11, 13, 14])
+def test_plain_short_segments_make_no_row_passes(n):
+    """One dense gate, or two that touch half of the entries, as two launches a
+    primitive; many gates on resident rows."""
+    import dmsim_amd as dm
+    for gates, launches in (([("H", [n - 1])], 2), ([("CX", [1, 0])], 2),
+                            ([("T", [0]), ("CX", [0, n - 1])], 4), ([("H", [0])] * 12, 3)):
+        t = W.GateTable(n)
+        for name, q in gates:
+            t.add(name, q)
+        s = dm.Sim(n)
+        s.append_table(t)
+        s.upload()
+        s.run()
+        assert s.last_run_stats()["launches"] == launches, gates
+        s.close()
