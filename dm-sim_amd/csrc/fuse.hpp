@@ -190,6 +190,19 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
 // most four qubits to a block.
 bool resident_wanted(const std::vector<Gate>& circuit, int n, int max_k);
 
+// Whether a resident plan of so many blocks is better off as sweeps.  From 9 qubits the
+// resident passes' two launches (and from 10 the conjugate transpose between them)
+// take 30, 41 and 78 us a run with one block and 32, 45 and 85 with two (9, 10 and
+// 11 qubits) where one sweep takes 24, 24 and 45 and two take 25, 42 to 46 and 79 to
+// 82; three take 34, 52 and 113 against 33, 49 and 98 to 99.  Below, one graph launch
+// hides the difference (24 us either way).
+inline bool resident_is_brief(int n, int blocks) { return n >= 9 && blocks <= 2; }
+
+// The tile width of such sweeps without a cost model, fastest on circuits of two blocks
+// (us a run at widths 6, 7 and 8): 9 qubits 26.5, 27.7 and 33; 10: 46, 36 and 43; 11: 110,
+// 85 and 81.  Timing the widths at upload would gain up to 2 us a run for 0.5 to 2.5 ms.
+inline int brief_tile_bits(int n) { return n <= 9 ? 6 : n == 10 ? 7 : 8; }
+
 // Whether a circuit's Hermitian plan runs as group sweeps.  With channels, from
 // 12 qubits: a group holds their whole neighbourhood where a four-qubit block
 // with a channel on every gate fills up with channels (a 300-member 12-qubit

@@ -60,3 +60,40 @@ def test_plain_short_segments_make_no_row_passes(n):
         s.run()
         assert s.last_run_stats()["launches"] == launches, gates
         s.close()
+
+
+@pytest.mark.parametrize("learned", [False, True])
+@pytest.mark.parametrize("n", [8, 9, 10, 11])
+def test_fused_short_unitary_circuits_run_as_sweeps(n, learned):
+    """From 9 qubits a circuit of one or two blocks makes a sweep a block and keeps
+    rho's orientation; deeper ones (and all at 8) run on resident rows."""
+    import costdata
+    import dmsim_amd as dm
+    model = costdata.default_model() if learned else None
+    for gates, brief in ((1, True), (4, True), (200, False)):
+        t = W.random_mixed(4, gates, 50 + n, gate_set=["H", "U3", "CX", "RZ"]) if brief else \
+            W.random_mixed(n, gates, 50 + n, gate_set=["H", "U3", "CX", "RZ"])
+        s, ref = dm.Sim(n), dm.Sim(n)
+        for x in (s, ref):
+            x.append_table(t)
+        s.set_method(dm.METHOD_FUSED)
+        if model is not None:
+            s.set_cost_model(model)
+        s.upload()
+        ref.upload()
+        s.set_profiling(True)
+        for _ in range(2):
+            s.run()
+            ref.run()
+            assert ("k_resident" in s.profile()) == (not brief or n < 9), gates
+            assert s.last_run_stats()["launches"] <= 3
+            got, want = s.get_dm(), ref.get_dm()
+            assert max(np.abs(got[i] - want[i]).max() for i in (0, 1)) <= 1e-12, gates
+        if brief and n >= 9:
+            info = s.plan_info()
+            assert info["fused_blocks"] + info["plain_blocks"] == 1
+            assert info["plain_blocks"] or s.last_run_stats()["launches"] == 1
+        s.close()
+        ref.close()
+    if model is not None:
+        model.close()
