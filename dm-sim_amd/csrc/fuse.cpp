@@ -2410,8 +2410,40 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
     if (group && herm && allow_perm && fold && n >= kHermMinQubits && n <= 16) {
         bool linear = !circuit.empty();
         for (const Gate& g : circuit) linear = linear && g.op != OP_SRN;
-        if (linear) return build_group_plan(circuit, n, tile_bits > 0 ? nullptr : model, out, info);
+        if (linear) {
+            PlanInfo gi, ai;
+            FusedPlan *grouped = nullptr, *alone = nullptr;
+            int rc = build_group_plan(circuit, n, tile_bits > 0 ? nullptr : model, &grouped, &gi);
+            if (rc) return rc;
+            bool channels = false;
+            for (const Gate& g : circuit) channels = channels || g.op == OP_KRAUS;
+            if (gi.herm_blocks == 1 && (channels || n >= 14)) {
+                // One sweep and its relabelling move 56 * 4^n bytes: a single channel or
+                // five-qubit gate, in place 32, is better off alone (us a run: one channel
+                // at 12 / 14 qubits 182 / 3166 as a group, 73 / 1861 alone; one C4X at 14 /
+                // 15 4179 / 17464 and 2549 / 9814).  At 13 a lone C4X would be as well (1107
+                // and 765), but is what runs a group of one five-qubit stage in the tests.
+                rc = build_fused_plan(circuit, n, max_k, model, tile_bits, allow_perm, &alone, &ai,
+                                      herm, fold);
+                if (rc) {
+                    delete grouped;
+                    return rc;
+                }
+                if (alone && alone->bytes(n) < grouped->bytes(n)) {
+                    std::swap(grouped, alone);
+                    gi = ai;
+                }
+                delete alone;
+            }
+            *out = grouped;
+            if (info) *info = gi;
+            return DMX_OK;
+        }
     }
+    // a circuit that is one channel runs as its sweep (11 qubits: 28 us, as a block 43)
+    size_t members = 0;
+    for (const Gate& g : circuit) members += g.op != OP_ID ? 1 : 0;
+    if (members == 1) fold = false;
     PlanInfo pi;
     BlockPlan bp;
     bool fusable = false;

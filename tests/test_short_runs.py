@@ -97,3 +97,32 @@ def test_fused_short_unitary_circuits_run_as_sweeps(n, learned):
         ref.close()
     if model is not None:
         model.close()
+
+
+@pytest.mark.parametrize("n,gate,kernel", [(8, None, "k_quad"), (11, None, "k_quad"), (12, None, "k_quad"),
+                                           (14, None, "k_quad"), (14, "C4X", "k_fused5")])
+def test_a_lone_channel_or_wide_gate_runs_in_place(n, gate, kernel):
+    """One launch in place, without a block or a group sweep around it."""
+    import dmsim_amd as dm
+    t = W.GateTable(n)
+    for q in range(n):
+        t.add("U3", [q], (0.3 + q, 0.2 * q, 0.7))
+    ref, s = dm.Sim(n), dm.Sim(n)
+    for x in (ref, s):  # a state first, then the circuit
+        x.append_table(t)
+        x.upload()
+        x.run()
+        x.clear_circuit()
+        if gate:
+            x.append(W.OP[gate], [0, 3, 5, 7, n - 1])
+        else:
+            x.append_kraus(n // 2, dm.amplitude_damping(0.3))
+    s.set_method(dm.METHOD_FUSED)
+    s.set_profiling(True)
+    idx = np.random.default_rng(n).integers(0, 4 ** n, size=4096, dtype=np.uint64)
+    for x in (ref, s):
+        x.upload()
+        x.run()
+    assert list(s.profile()) == [kernel] and s.last_run_stats()["launches"] == 1
+    assert np.abs(s.get_entries(idx) - ref.get_entries(idx)).max() <= 1e-12
+    assert np.abs(s.get_diag() - ref.get_diag()).max() <= 1e-12
