@@ -479,7 +479,9 @@ int Batch::upload()
                         if (s < circs_[i].n_blocks && circs_[i].resident) {
                             const bool flip = circs_[i].n_blocks == 3;
                             const int kind = s == 0 || s == 2 ? SK_ROWS : flip ? SK_FLIP : SK_COLUMNS;
-                            by[{resident_log_entries(circs_[i].n), kind, 0}].push_back(i);
+                            by[{resident_log_entries(circs_[i].n), kind,
+                                resident_extra(circs_[i].n, kind == SK_COLUMNS)}]
+                                .push_back(i);
                         } else if (s < circs_[i].n_blocks) {
                             const size_t b = circs_[i].blk_off + s;
                             const int kind = kinds_[b];
@@ -500,7 +502,8 @@ int Batch::upload()
                             std::stable_sort(kv.second.begin(), kv.second.end(), [&](int a, int b) {
                                 return circs_[a].job.blocks > circs_[b].job.blocks;
                             });
-                            lst.push_back(Launch{L, 0, (int)kv.second.size(), jobs.size(), w, kind});
+                            lst.push_back(Launch{L, std::get<2>(kv.first), (int)kv.second.size(),
+                                                 jobs.size(), w, kind});
                             for (int i : kv.second) jobs.push_back(circs_[i].job);
                             continue;
                         }
@@ -732,7 +735,7 @@ hipError_t Batch::launch(const Launch& l, const BatchEntry* d_entries)
         return launch_conj_transpose(j.re, j.im, j.n, stream_);
     }
     if (l.kind == SK_ROWS || l.kind == SK_COLUMNS)
-        return launch_resident_batch(d_res_jobs_ + l.entry_off, l.count, l.n, l.kind == SK_COLUMNS,
+        return launch_resident_batch(d_res_jobs_ + l.entry_off, l.count, l.n, l.kind == SK_COLUMNS, l.m,
                                      stream_);
     const BatchEntry* e = d_entries + l.entry_off;
     switch (l.kind) {

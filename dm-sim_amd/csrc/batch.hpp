@@ -155,7 +155,7 @@ private:
     };
     struct Launch {
         int n;
-        int m;
+        int m;  // (resident columns: resident_extra)
         int count;
         size_t entry_off;  // into the entries, or (resident) the jobs
         int wave;

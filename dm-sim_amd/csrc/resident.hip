@@ -37,19 +37,22 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c)
 
 }  // namespace
 
-// n <= LOGE; a chunk is 2^LOGE entries, 2^(LOGE - 8) tiles, dealt to the waves
-// in runs.  SLOW: rows and columns of rho exchanged, and conjugated values.
-template <int LOGE, int WAVES, bool SLOW>
+// n <= LOGE; a chunk is 2^C entries, C = LOGE + X, in 2^(C - 8) tiles, dealt to the
+// waves in runs.  SLOW: rows and columns of rho exchanged, and conjugated values.  X: as
+// many rows more to a chunk as records of 2^LOGE entries have tiles (2^X times), so that
+// a SLOW one's columns lie together in memory.
+template <int LOGE, int WAVES, bool SLOW, int X = 0>
 __device__ __forceinline__ void resident_pass(const ResidentJob& job)
 {
+    constexpr int C = LOGE + X;
     double* const re = job.re;
     double* const im = job.im;
     const double2* const parts = reinterpret_cast<const double2*>(job.parts);
     const int blocks = job.blocks, n = job.n;
     const ResidentEnd& end = job.end;
     constexpr int kThreads = 64 * WAVES;
-    constexpr int kPer = (1 << (LOGE - 8)) / WAVES;  // tiles of a wave
-    __shared__ double2 s[1 << LOGE];
+    constexpr int kPer = (1 << (C - 8)) / WAVES;  // tiles of a wave
+    __shared__ double2 s[1 << C];
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u, wave = tid >> 6;
     // entry i of the thread's share in memory order: its index in the chunk, its offset
@@ -57,9 +60,9 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
         const uint32_t f = SLOW ? tid + i * kThreads : 2 * (tid + i * kThreads);
         if constexpr (!SLOW) {
             e = f;
-            return ((uint64_t)blockIdx.x << LOGE) + f;
+            return ((uint64_t)blockIdx.x << C) + f;
         }
-        const int rows = LOGE - n;  // 2^rows columns of rho to a chunk, neighbours together
+        const int rows = C - n;  // 2^rows columns of rho to a chunk, neighbours together
         const uint32_t c = f & ((1u << rows) - 1u), r = f >> rows;
         e = r | c << n;
         return ((uint64_t)r << n) + ((uint64_t)blockIdx.x << rows) + c;
@@ -72,19 +75,19 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
 
     if constexpr (SLOW) {
 #pragma unroll
-        for (int i = 0; i < (1 << LOGE) / kThreads; i++) {
+        for (int i = 0; i < (1 << C) / kThreads; i++) {
             uint32_t e;
             const uint64_t off = entry(i, e);
-            s[row_place(e, 3, LOGE)] = make_double2(re[off], -im[off]);
+            s[row_place(e, 3, C)] = make_double2(re[off], -im[off]);
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < (1 << LOGE) / kThreads / 2; i++) {
+        for (int i = 0; i < (1 << C) / kThreads / 2; i++) {
             uint32_t e;
             const uint64_t off = entry(i, e);
             const double2 r = *reinterpret_cast<const double2*>(re + off);
             const double2 m = *reinterpret_cast<const double2*>(im + off);
-            const uint32_t x = row_place(e, 3, LOGE);
+            const uint32_t x = row_place(e, 3, C);
             s[x] = make_double2(r.x, m.x);
             s[x ^ 1u] = make_double2(r.y, m.y);
         }
@@ -109,6 +112,8 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
             uint32_t x[4] = {w0 & 0xFFFFu};
 #pragma unroll
             for (int i = 0; i < LOGE - 8; i++) x[0] ^= (tile >> i) & 1u ? t[i] : 0u;
+#pragma unroll
+            for (int i = LOGE; i < C; i++) x[0] ^= (tile >> (i - 8)) & 1u ? row_place(1u << i, 3, C) : 0u;
             x[1] = x[0] ^ c0;
             x[2] = x[0] ^ c1;
             x[3] = x[1] ^ c1;
@@ -137,11 +142,13 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
         uint32_t x = end.base;
 #pragma unroll
         for (int i = 0; i < LOGE; i++) x ^= (e >> i) & 1u ? end.bit[i] : 0u;
+#pragma unroll
+        for (int i = LOGE; i < C; i++) x ^= (e >> i) & 1u ? row_place(1u << i, 3, C) : 0u;
         return x;
     };
     if constexpr (SLOW) {
 #pragma unroll
-        for (int i = 0; i < (1 << LOGE) / kThreads; i++) {
+        for (int i = 0; i < (1 << C) / kThreads; i++) {
             uint32_t e;
             const uint64_t off = entry(i, e);
             const double2 v = s[end_place(e)];
@@ -150,7 +157,7 @@ __device__ __forceinline__ void resident_pass(const ResidentJob& job)
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < (1 << LOGE) / kThreads / 2; i++) {
+        for (int i = 0; i < (1 << C) / kThreads / 2; i++) {
             uint32_t e;
             const uint64_t off = entry(i, e);
             const uint32_t x = end_place(e);
@@ -167,12 +174,12 @@ __global__ void __launch_bounds__(64 * WAVES, 5) k_resident(const ResidentJob jo
     resident_pass<LOGE, WAVES, SLOW>(job);
 }
 
-template <int LOGE, int WAVES, bool SLOW>
+template <int LOGE, int WAVES, bool SLOW, int X = 0>
 __global__ void __launch_bounds__(64 * WAVES, 5) k_resident_batch(const ResidentJob* __restrict__ jobs)
 {
     const ResidentJob& job = jobs[blockIdx.y];
-    if (blockIdx.x >= 1u << (2 * job.n - LOGE)) return;  // a narrower circuit's
-    resident_pass<LOGE, WAVES, SLOW>(job);
+    if (blockIdx.x >= 1u << (2 * job.n - LOGE - X)) return;  // a narrower circuit's
+    resident_pass<LOGE, WAVES, SLOW, X>(job);
 }
 
 hipError_t launch_resident(const ResidentJob& job, bool slow, hipStream_t stream)
@@ -194,19 +201,22 @@ hipError_t launch_resident(const ResidentJob& job, bool slow, hipStream_t stream
 }
 
 hipError_t launch_resident_batch(const ResidentJob* d_jobs, int count, int log_entries, bool slow,
-                                 hipStream_t stream)
+                                 int extra, hipStream_t stream)
 {
     if (count < 1 || count > 65535 || log_entries < 8 ||
         log_entries > (slow ? kResidentColumnQubits : kResidentMaxQubits))
         return hipErrorInvalidValue;
-    const dim3 grid(1u << log_entries, (unsigned)count);  // n = log_entries has the most chunks
-    switch (2 * log_entries + (slow ? 1 : 0)) {
+    const dim3 grid(1u << (log_entries - extra), (unsigned)count);  // n = log_entries: most chunks
+    switch (100 * extra + 2 * log_entries + (slow ? 1 : 0)) {
     case 16: k_resident_batch<8, 1, false><<<grid, 64, 0, stream>>>(d_jobs); break;
     case 17: k_resident_batch<8, 1, true><<<grid, 64, 0, stream>>>(d_jobs); break;
+    case 117: k_resident_batch<8, 2, true, 1><<<grid, 128, 0, stream>>>(d_jobs); break;
+    case 317: k_resident_batch<8, 8, true, 3><<<grid, 512, 0, stream>>>(d_jobs); break;
     case 18: k_resident_batch<9, 2, false><<<grid, 128, 0, stream>>>(d_jobs); break;
-    case 19: k_resident_batch<9, 2, true><<<grid, 128, 0, stream>>>(d_jobs); break;
+    case 319: k_resident_batch<9, 8, true, 3><<<grid, 512, 0, stream>>>(d_jobs); break;
     case 20: k_resident_batch<10, 4, false><<<grid, 256, 0, stream>>>(d_jobs); break;
-    default: k_resident_batch<11, 4, false><<<grid, 256, 0, stream>>>(d_jobs); break;
+    case 22: k_resident_batch<11, 4, false><<<grid, 256, 0, stream>>>(d_jobs); break;
+    default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }

@@ -65,9 +65,18 @@ struct ResidentJob {
 // slow (n <= kResidentColumnQubits): rho <- conj(U) rho.  In place.
 hipError_t launch_resident(const ResidentJob& job, bool slow, hipStream_t stream);
 
+// A batch's column passes run together and stream from memory, where a column alone is
+// a strided run of 8-byte accesses: chunks take 2^X times as many columns (extra = X), 64
+// bytes side by side at 8 and 9 qubits, 32 at 7.  96 ansatz circuits of 1 / 9 layers, us
+// a run with X = 0, 1, 2, 3: 7 qubits 91 / 121, 69 / 110, -, 87 / 189 (waves that
+// wait for one another's tiles); 8: 394 / 496, -, 180 / 357, 143 / 353; 9: 1497 / 1887, -,
+// 853 / 1394, 572 / 1293; 6: 51 / 66 and 76 / 132 with 0 and 3.
+inline int resident_extra(int n, bool slow) { return !slow || n < 7 ? 0 : n == 7 ? 1 : 3; }
+
 // The same for `count` circuits whose chunks have 2^log_entries entries
-// (resident_log_entries of every job's n, so one launch takes all widths up to 8).
+// (resident_log_entries of every job's n, so one launch takes all widths up to 8), times
+// 2^extra (resident_extra of every job's n).
 hipError_t launch_resident_batch(const ResidentJob* d_jobs, int count, int log_entries, bool slow,
-                                 hipStream_t stream);
+                                 int extra, hipStream_t stream);
 
 }  // namespace dmx

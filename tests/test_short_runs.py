@@ -126,3 +126,31 @@ def test_a_lone_channel_or_wide_gate_runs_in_place(n, gate, kernel):
     assert list(s.profile()) == [kernel] and s.last_run_stats()["launches"] == 1
     assert np.abs(s.get_entries(idx) - ref.get_entries(idx)).max() <= 1e-12
     assert np.abs(s.get_diag() - ref.get_diag()).max() <= 1e-12
+
+
+@pytest.mark.parametrize("n", [5, 6, 7, 8, 9])
+def test_batched_column_passes_equal_single_runs(n):
+    """Column passes of several columns to a chunk (7 to 9 qubits), more circuits than one,
+    of uneven depth and beside other widths: bit for bit the circuits' own runs."""
+    import dmsim_amd as dm
+    rng = np.random.default_rng(n)
+    widths = [n, n, 6, n, 8, n]
+    circuits = [W.random_mixed(w, int(rng.integers(60, 300)), 20 * n + i,
+                               gate_set=["H", "U3", "CX", "SWAP", "X", "RZZ", "CCX"])
+                for i, w in enumerate(widths)]
+    b = dm.Batch()
+    for t in circuits:
+        b.add_circuit(t)
+    b.upload()
+    for _ in range(2):
+        b.run()
+    for i, t in enumerate(circuits):
+        s = dm.Sim(t.n_qubits)
+        s.set_method(dm.METHOD_FUSED)
+        s.append_table(t)
+        s.upload()
+        s.run()
+        got, want = b.get_dm(i), s.get_dm()
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), i
+        s.close()
+    b.close()
