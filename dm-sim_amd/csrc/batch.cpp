@@ -218,7 +218,7 @@ int Batch::upload()
     kinds_.clear();
     for (Circ& c : circs_) {
         c.plan.reset();
-        c.solo = c.herm = c.resident = false;
+        c.solo = c.herm = c.resident = c.brief = false;
         c.solo_launches = 0;
     }
     std::vector<FusedBlock> blocks;
@@ -278,6 +278,19 @@ int Batch::upload()
                 c.job = p->resident_job();
                 c.parts_off = parts.size();
                 parts.insert(parts.end(), p->resident_parts().begin(), p->resident_parts().end());
+                continue;
+            }
+            std::vector<PlanStepView> steps;
+            if (p) p->describe(steps);
+            if (!steps.empty()) {  // too few blocks: in place, at the default width
+                for (const PlanStepView& v : steps) {
+                    blocks.push_back(*v.block);
+                    blocks.back().m = (uint32_t)default_tile_bits(c.n);
+                    kinds.push_back((uint8_t)SK_INORDER);
+                }
+                c.brief = true;
+                c.n_blocks = steps.size();
+                c.bytes = (double)c.n_blocks * sweep;
                 continue;
             }
         }
@@ -431,7 +444,9 @@ int Batch::upload()
     };
     if (!blocks.empty()) BTRY(hipMalloc(&d_blocks_, blocks.size() * sizeof(FusedBlock)));
     for (const Circ& c : circs_) tile_bits_[c.n] = default_tile_bits(c.n);
-    if (autotune_ && !blocks.empty()) {
+    bool timed = false;  // sweeps whose widths and groups are timed (not brief ones)
+    for (const Circ& c : circs_) timed = timed || (!c.solo && !c.resident && !c.brief && c.n_blocks > 0);
+    if (autotune_ && timed) {
         BTRY(hipMemcpy(d_blocks_, blocks.data(), blocks.size() * sizeof(FusedBlock),
                        hipMemcpyHostToDevice));
         const int rc = autotune(blocks);
@@ -519,7 +534,7 @@ int Batch::upload()
     };
     if (!group_fixed_) {
         group_bytes_ = 0;
-        if (autotune_ && !blocks.empty()) {
+        if (autotune_ && timed) {
             const int rc = autotune_groups(build);
             if (rc) return rc;
         }
@@ -617,7 +632,8 @@ int Batch::autotune(std::vector<FusedBlock>& blocks)
 {
     std::map<int, std::vector<int>> by_n;  // circuits of in-order blocks by qubit count
     for (int i = 0; i < (int)circs_.size(); i++)
-        if (circs_[i].n_blocks > 0 && !circs_[i].herm && !circs_[i].resident) by_n[circs_[i].n].push_back(i);
+        if (circs_[i].n_blocks > 0 && !circs_[i].herm && !circs_[i].resident && !circs_[i].brief)
+            by_n[circs_[i].n].push_back(i);
     if (by_n.empty()) return DMX_OK;
     BTRY(hipMemsetAsync(pool_, 0, pool_doubles_ * sizeof(double), stream_));
     size_t most = 0;
@@ -666,7 +682,7 @@ int Batch::autotune(std::vector<FusedBlock>& blocks)
     (void)hipFree(d_tmp);
     if (rc) return rc;
     for (const Circ& c : circs_)
-        if (!c.herm && !c.resident)
+        if (!c.herm && !c.resident && !c.brief)
             for (size_t b = 0; b < c.n_blocks; b++)
                 blocks[c.blk_off + b].m = (uint32_t)tile_bits_[c.n];
     return DMX_OK;

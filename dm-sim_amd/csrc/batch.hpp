@@ -131,6 +131,7 @@ private:
         std::vector<Gate> gates;  // C4X expanded (batched blocks have at most four qubits)
         bool solo = false;        // runs on its own (kSoloQubits and up)
         bool resident = false;    // its blocks run on resident rows
+        bool brief = false;       // too few of them for that: sweeps at the default width
         size_t parts_off = 0;     // its records
         ResidentJob job = {};
         bool herm = false;        // its batched steps are Hermitian sweeps and relabellings

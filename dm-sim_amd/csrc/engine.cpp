@@ -164,34 +164,17 @@ int Engine::upload()
         // the settings that ask for a form of sweep keep the sweeps
         const bool resident = fusion_permute_ && fusion_herm_ == 1 && tile_bits_ == 0 &&
                               resident_wanted(circuit_, n_, fusion_max_k_);
-        int width = tile_bits_;  // of every sweep; 0: chosen
-        int rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, width, fusion_permute_, &plan_,
-                                  &plan_info_, herm, fold, group_wanted(circuit_, n_), resident);
+        int rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_,
+                                  fusion_permute_, &plan_, &plan_info_, herm, fold,
+                                  group_wanted(circuit_, n_), resident);
         if (rc) return rc;
-        if (plan_ && plan_->resident() && resident_is_brief(n_, plan_->resident_job().blocks)) {
-            // a plan this short as sweeps, if it is as short there (other groupings)
-            if (!model_) width = brief_tile_bits(n_);  // timing the widths costs hundreds of runs
-            FusedPlan* sweeps = nullptr;
-            PlanInfo si;
-            rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, width, fusion_permute_, &sweeps,
-                                  &si, herm, fold, false, false);
-            if (rc) return rc;
-            if (sweeps && resident_is_brief(n_, (int)(si.fused_blocks + si.plain_blocks))) {
-                delete plan_;
-                plan_ = sweeps;
-                plan_info_ = si;
-            } else {
-                delete sweeps;
-                width = tile_bits_;
-            }
-        }
         if (plan_ && !plan_->resident() && plan_info_.perm_blocks > 0 && n_ < kPermuteSureQubits && fusion_herm_ != 2) {
             // a short sweep is latency-bound and a permuting one pays its index
             // map's set-up: keep the permuting plan only if it still wins
             FusedPlan* inplace = nullptr;
             PlanInfo ii;
-            rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, width, false, &inplace, &ii,
-                                  false, fold);
+            rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_, false,
+                                  &inplace, &ii, false, fold);
             if (rc) return rc;
             if (inplace && !permuting_pays(plan_info_, ii)) {
                 drop_graph();
@@ -218,8 +201,8 @@ int Engine::upload()
                 drop_graph();
                 delete plan_;
                 plan_ = nullptr;
-                rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, width, false, &plan_,
-                                      &plan_info_, false, fold);
+                rc = build_fused_plan(circuit_, n_, fusion_max_k_, model_, tile_bits_, false,
+                                      &plan_, &plan_info_, false, fold);
                 if (rc) return rc;
             }
         }
@@ -227,8 +210,8 @@ int Engine::upload()
             rc = plan_->upload(stream_);
             if (rc) return rc;
             tuned_tile_bits_ = 0;
-            if (!model_ && width == 0 && fusion_autotune_ && plan_info_.herm_blocks == 0 &&
-                !plan_->resident()) {
+            if (!model_ && tile_bits_ == 0 && fusion_autotune_ && plan_info_.herm_blocks == 0 &&
+                !resident) {
                 // the greedy plan's tile width, measured: on the second pair of
                 // planes if there is one, else on scratch planes (rho untouched)
                 double *sr = d_re2_, *si = d_im2_;

@@ -2509,7 +2509,20 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
             plan->steps.push_back({ST_PLAIN, first, (int)plan->prims.size() - first});
         }
     }
-    if (resident) plan->make_resident();
+    if (resident) {
+        bool brief = resident_is_brief(n, (int)plan->steps.size());
+        for (const FusedBlock& fb : plan->blocks) brief = brief && !fb.perm_on;
+        if (brief) {  // the same blocks in place
+            std::memset(pi.tile_hist, 0, sizeof(pi.tile_hist));
+            for (FusedBlock& fb : plan->blocks) {
+                fb.m = (uint32_t)(tile_bits_ok(n, brief_tile_bits(n), fb.qmask) ? brief_tile_bits(n)
+                                                                                 : default_tile_bits(n));
+                pi.tile_hist[fb.m]++;
+            }
+        } else {
+            plan->make_resident();
+        }
+    }
     if (herm) to_hermitian(*plan, n, pi);
     if (herm && model && tile_bits <= 0) {
         rc = reprice_fused5_widths(*plan, n, *model);

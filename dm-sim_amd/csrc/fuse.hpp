@@ -190,18 +190,24 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
 // most four qubits to a block.
 bool resident_wanted(const std::vector<Gate>& circuit, int n, int max_k);
 
-// Whether a resident plan of so many blocks is better off as sweeps.  From 9 qubits the
-// resident passes' two launches (and from 10 the conjugate transpose between them)
-// take 30, 41 and 78 us a run with one block and 32, 45 and 85 with two (9, 10 and
-// 11 qubits) where one sweep takes 24, 24 and 45 and two take 25, 42 to 46 and 79 to
-// 82; three take 34, 52 and 113 against 33, 49 and 98 to 99.  Below, one graph launch
-// hides the difference (24 us either way).
-inline bool resident_is_brief(int n, int blocks) { return n >= 9 && blocks <= 2; }
+// Whether a resident plan of so many blocks, none with a trailing permutation, runs them as
+// in-place sweeps after all.  Alone, from 9 qubits the resident passes' two launches (and
+// from 10 the conjugate transpose between them) take 30, 41 and 78 us a run with one block
+// and 32, 45 and 85 with two (9, 10 and 11 qubits) where one sweep takes 21, 22 and 45 and two
+// take 25, 41 and 79 to 83; three take 34, 52 and 113 against 33, 49 and 98.  Below 9 one
+// graph launch hides the difference (20 to 24 us either way up to two, 26 against 21 with
+// three).  In a batch (96 circuits of 4 to 9 qubits, 64 of 10, 32 of 11) one block takes 37, 39,
+// 46, 64, 112, 488, 1651 and 3145 us resident and 26, 24, 29, 50, 91, 295, 696 and 1330 in
+// place; two 45 and 51 against 30 and 39 (5 and 6 qubits); three, from 7 to 11, 72, 144,
+// 573, 1874 and (four) 3796 against 91, 208, 710, 1622 and 4055.  One rule for both, so
+// that a batched rho stays bit-identical to the circuit's own run.  At 4 qubits, where a
+// plan is one block, alone both take 24 us, and the resident form is what a test of it runs.
+inline bool resident_is_brief(int n, int blocks) { return n > 4 && blocks <= 2; }
 
-// The tile width of such sweeps without a cost model, fastest on circuits of two blocks
-// (us a run at widths 6, 7 and 8): 9 qubits 26.5, 27.7 and 33; 10: 46, 36 and 43; 11: 110,
-// 85 and 81.  Timing the widths at upload would gain up to 2 us a run for 0.5 to 2.5 ms.
-inline int brief_tile_bits(int n) { return n <= 9 ? 6 : n == 10 ? 7 : 8; }
+// The tile width of such sweeps of one circuit, fastest on circuits of two blocks (us a run at
+// widths 6, 7 and 8): 8 qubits 20.4, 23.4 and 30; 9 26.5, 27.7 and 33; 10 46, 36 and 43; 11
+// 110, 85 and 81.  Timing the widths at upload would gain up to 2 us a run for 0.5 to 2.5 ms.
+inline int brief_tile_bits(int n) { return n < 6 ? n : n <= 9 ? 6 : n == 10 ? 7 : 8; }
 
 // Whether a circuit's Hermitian plan runs as group sweeps.  With channels, from
 // 12 qubits: a group holds their whole neighbourhood where a four-qubit block

@@ -63,10 +63,10 @@ def test_plain_short_segments_make_no_row_passes(n):
 
 
 @pytest.mark.parametrize("learned", [False, True])
-@pytest.mark.parametrize("n", [8, 9, 10, 11])
+@pytest.mark.parametrize("n", [5, 8, 9, 10, 11])
 def test_fused_short_unitary_circuits_run_as_sweeps(n, learned):
-    """From 9 qubits a circuit of one or two blocks makes a sweep a block and keeps
-    rho's orientation; deeper ones (and all at 8) run on resident rows."""
+    """A circuit of one or two blocks makes a sweep a block and keeps rho's orientation;
+    deeper ones run on resident rows."""
     import costdata
     import dmsim_amd as dm
     model = costdata.default_model() if learned else None
@@ -85,11 +85,11 @@ def test_fused_short_unitary_circuits_run_as_sweeps(n, learned):
         for _ in range(2):
             s.run()
             ref.run()
-            assert ("k_resident" in s.profile()) == (not brief or n < 9), gates
+            assert ("k_resident" in s.profile()) != brief, gates
             assert s.last_run_stats()["launches"] <= 3
             got, want = s.get_dm(), ref.get_dm()
             assert max(np.abs(got[i] - want[i]).max() for i in (0, 1)) <= 1e-12, gates
-        if brief and n >= 9:
+        if brief:
             info = s.plan_info()
             assert info["fused_blocks"] + info["plain_blocks"] == 1
             assert info["plain_blocks"] or s.last_run_stats()["launches"] == 1
@@ -154,3 +154,40 @@ def test_batched_column_passes_equal_single_runs(n):
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), i
         s.close()
     b.close()
+
+
+def test_batched_short_circuits_equal_single_runs():
+    """Circuits of one or two blocks beside deeper ones, 4 to 11 qubits, in one wave and in
+    several: bit for bit the circuits' own runs, without a second pool of planes."""
+    import dmsim_amd as dm
+    rng = np.random.default_rng(8)
+    circuits = []
+    for n in range(4, 12):
+        circuits.append(W.GateTable(n).add("RY", [n - 1], (0.7, 0, 0)))
+        circuits.append(W.random_mixed(min(n, 6), 12, 60 + n, gate_set=["H", "CX", "U3", "SWAP", "X"]))
+        circuits[-1].n_qubits = n
+        circuits.append(W.hea_circuit(n, 5, rng))
+    want = []
+    for t in circuits:
+        s = dm.Sim(t.n_qubits)
+        s.set_method(dm.METHOD_FUSED)
+        s.append_table(t)
+        s.upload()
+        s.run()
+        want.append((s.get_diag(), *s.get_dm()))
+        s.close()
+    for limit in (0, 16 << 22):
+        b = dm.Batch()
+        b.set_pool_limit(limit)
+        for t in circuits:
+            b.add_circuit(t)
+        b.upload()
+        assert limit == 0 or b.waves() > 1
+        for _ in range(3):
+            b.run()
+        for i, (diag, re, im) in enumerate(want):
+            assert np.array_equal(b.get_diag(i), diag), i
+            if limit == 0 and circuits[i].n_qubits < 10:
+                got = b.get_dm(i)
+                assert np.array_equal(got[0], re) and np.array_equal(got[1], im), i
+        b.close()
