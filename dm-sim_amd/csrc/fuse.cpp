@@ -1371,8 +1371,10 @@ struct StageSpec {
     uint32_t kind;   // GroupStageKind
     uint32_t mask;   // the qubits it acts on
     std::vector<int> members;
-    double cost() const { return kind == GS_UNITARY5 ? 2.0 : kind == GS_PAIR ? 0.5 : 1.0; }  // in 24 MFMAs
-                                                                                            // per 256 entries
+    double cost() const  // in 24 MFMAs per 256 entries
+    {
+        return kind == GS_UNITARY5 ? 2.0 : kind == GS_PAIR ? 16.0 / 24.0 : 1.0;
+    }
 };
 
 // Channel-free members as unitaries of four bits, each member joining the one
@@ -2168,11 +2170,11 @@ int reprice_fused5_widths(Plan& plan, int n, CostModel& model)
 
 // Predicted time of one group sweep with stages of the given cost (StageSpec),
 // base = a four-qubit Hermitian sweep's as the network prices it on the lowest
-// bits.  Fitted at 14 qubits (base 977 us): 1141 us with one stage, 1571 with
-// 2.17 on average, 1600 with 2.41.
+// bits.  Fitted at 14 qubits (base 977 us): 1689 us with 2.17 stages on average; with
+// one, about 1.2 times the base.
 double group_us(double base, double stage_cost)
 {
-    return base * (0.79 + 0.376 * stage_cost);
+    return base * (0.79 + 0.43 * stage_cost);
 }
 
 // Grouping into group sweeps: without a model, the frontier search with its

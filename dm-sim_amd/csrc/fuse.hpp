@@ -216,9 +216,9 @@ inline int brief_tile_bits(int n) { return n < 6 ? n : n <= 9 ? 6 : n == 10 ? 7 
 // its launch).  With five-qubit gates, from 13: the five-qubit sweep has no
 // Hermitian form (structured circuits 20.3 -> 14.3 ms at 13 qubits, 77 -> 62.5
 // at 14, 332 -> 289 at 15).  Other unitary circuits keep four-qubit sweeps: on
-// 2130 gates at 14 qubits 116 group sweeps of 1.57 ms take 182 ms, 181 of the
-// others 177, as a group's 2.2 stages occupy the matrix cores for 1.15 ms that
-// overlap its 1.1 ms of memory traffic only in part.
+// 2130 gates at 14 qubits 113 group sweeps of 1.69 ms take 193 ms, 181 of the
+// others 177, as a group's 2.2 stages occupy the matrix cores for 1 ms that
+// overlaps its 1.1 ms of memory traffic only in part.
 bool group_wanted(const std::vector<Gate>& circuit, int n);
 
 // From this many qubits the engine folds channels into blocks.  A noisy

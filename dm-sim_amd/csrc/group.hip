@@ -8,11 +8,11 @@
 // its stages run (not where a five-qubit stage needs the registers).
 //
 // Bound by both memory and matrix cores: on 14 qubits a sweep without stages
-// takes 1150 us (4.3 GB, 3.7 TB/s), the stages alone 135 us + 430 us per
-// four-qubit stage (24 MFMAs of 2048 operations per 256 entries: 64 of the
-// 65-67 TFLOP/s that a long run of these instructions reaches); a sweep with 2.4
-// stages 1600 us.  512 threads, i.e. four waves per SIMD, took 1880 us: the matrix
-// core is as busy with two, and each wave's stage setup counts twice.
+// takes 1150 us (4.3 GB, 3.7 TB/s) and a four-qubit stage keeps the matrix cores busy
+// for 430 us (24 MFMAs of 2048 operations per 256 entries, at 64 of the 65-67
+// TFLOP/s that a long run of these instructions reaches); a sweep with 2.2 stages on
+// average 1690 us.  512 threads, i.e. four waves per SIMD, took longer: the matrix core
+// is as busy with two, and each wave's stage setup counts twice.
 #include <hip/hip_runtime.h>
 
 #include "group.hpp"
@@ -34,11 +34,13 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c)
 constexpr uint32_t kMatsInLds = 2048;
 
 // MFMA lane layout: A[i][k] in lane i + 16k, B[k][j] in lane j + 16k, D[4r + g][j]
-// in lane j + 16g register r.  A complex product takes three real ones, arranged
-// so that the accumulators do the additions: with K = (Ar + Ai) Br,
-// re = K - Ai (Br + Bi) and im = K + Ar (Bi - Br), both chains starting from K.
-// (FP64 additions on the vector unit wait for the matrix core: 558 -> 519 us per
-// stage of a 14-qubit sweep against combining three separate products.)
+// in lane j + 16g register r.  Complex products round as those of the block sweeps
+// do: unitaries take three real products combined after their sums, superoperators four.
+// Chaining three through one sum (re = K - Ai (Br + Bi), im = K + Ar (Bi - Br) from K = (Ar +
+// Ai) Br) lets the accumulators do the additions and is faster where a sweep has
+// several stages (2.2 on average at 14 qubits 1577 us for 1689; 40 noisy gates at 12 qubits
+// 1350 us a run for 1520), but further off: RMS over rho after those 40 gates 1.76e-15
+// for 1.52e-15, where one sweep per channel has 1.58e-15.
 
 // A unitary on four bits: 16 sub-tiles of 16 x 16 (the other two bits of rows
 // and columns), wave w those with row part w, two at a time; per sub-tile X =
@@ -50,14 +52,12 @@ __device__ __forceinline__ void stage_unitary4(const GroupStage& s, const Mat& m
                                                int kk, double* __restrict__ s_re,
                                                double* __restrict__ s_im)
 {
-    double ur[4], us[4], ud[4];
+    double ur[4], ui[4];
     uint32_t urow[4], ucol[4];  // places of matrix index 4c as a row, as a column
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        const double ui = mat(256 + j * 16 + 4 * c + kk);
         ur[c] = mat(j * 16 + 4 * c + kk);
-        us[c] = ur[c] + ui;
-        ud[c] = ur[c] - ui;
+        ui[c] = mat(256 + j * 16 + 4 * c + kk);
         const uint32_t q = group_local(s, 2, 2, c);
         urow[c] = group_row_place(q);
         ucol[c] = group_col_place(q);
@@ -78,38 +78,37 @@ __device__ __forceinline__ void stage_unitary4(const GroupStage& s, const Mat& m
                 ti[u][c] = s_im[rd ^ (base[u] ^ ucol[c])];
             }
         }
-        d4 k[2] = {}, xr[2], xi[2], yr[2], yi[2];
+        d4 p[2] = {}, q[2] = {}, k[2] = {}, xr[2], xi[2];
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int u = 0; u < 2; u++) k[u] = mfma(tr[u][c] + ti[u][c], ur[c], k[u]);
+            for (int u = 0; u < 2; u++) {
+                p[u] = mfma(tr[u][c], ur[c], p[u]);
+                q[u] = mfma(ti[u][c], ui[c], q[u]);
+                k[u] = mfma(tr[u][c] + ti[u][c], ur[c] + ui[c], k[u]);
+            }
 #pragma unroll
         for (int u = 0; u < 2; u++) {
-            xr[u] = xi[u] = k[u];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                xr[u] = mfma(ti[u][c], -us[c], xr[u]);
-                xi[u] = mfma(tr[u][c], -ud[c], xi[u]);
-            }
-            k[u] = d4{0, 0, 0, 0};
+            xr[u] = p[u] - q[u];
+            xi[u] = k[u] - p[u] - q[u];
+            p[u] = q[u] = k[u] = d4{0, 0, 0, 0};
         }
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int c = 0; c < 4; c++) k[u] = mfma(ur[c], xr[u][c] + xi[u][c], k[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            yr[u] = yi[u] = k[u];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                yr[u] = mfma(-ud[c], xi[u][c], yr[u]);
-                yi[u] = mfma(-us[c], xr[u][c], yi[u]);
+            for (int u = 0; u < 2; u++) {
+                p[u] = mfma(ur[c], xr[u][c], p[u]);
+                q[u] = mfma(-ui[c], xi[u][c], q[u]);
+                k[u] = mfma(ur[c] - ui[c], xr[u][c] + xi[u][c], k[u]);
             }
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const d4 yr = p[u] - q[u];
+            const d4 yi = k[u] - p[u] - q[u];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                s_re[wr ^ (base[u] ^ urow[r])] = yr[u][r];
-                s_im[wr ^ (base[u] ^ urow[r])] = yi[u][r];
+                s_re[wr ^ (base[u] ^ urow[r])] = yr[r];
+                s_im[wr ^ (base[u] ^ urow[r])] = yi[r];
             }
         }
     }
@@ -117,20 +116,18 @@ __device__ __forceinline__ void stage_unitary4(const GroupStage& s, const Mat& m
 
 // A superoperator of two bits: Y = S X with X's rows their 16 (row, column)
 // values and its columns 16 values of the other bits; wave w takes the other
-// row bits' values 4w..4w+3, two at a time (12 MFMAs each, read and written by the
+// row bits' values 4w..4w+3, two at a time (16 MFMAs each, read and written by the
 // same lane).
 template <class Mat>
 __device__ __forceinline__ void stage_pair(const GroupStage& s, const Mat& mat, int wave, int j, int kk,
                                            double* __restrict__ s_re, double* __restrict__ s_im)
 {
-    double ur[4], us[4], ud[4];
+    double ur[4], ui[4];
     uint32_t urow[4];
 #pragma unroll
     for (int c = 0; c < 4; c++) {
-        const double ui = mat(256 + j * 16 + 4 * c + kk);
         ur[c] = mat(j * 16 + 4 * c + kk);
-        us[c] = ur[c] + ui;
-        ud[c] = ui - ur[c];
+        ui[c] = mat(256 + j * 16 + 4 * c + kk);
         urow[c] = group_row_place(group_local(s, 0, 2, c));
     }
     const uint32_t lane = group_col_place(group_local(s, 0, 2, kk) | group_local(s, 2, 4, j));
@@ -147,25 +144,28 @@ __device__ __forceinline__ void stage_pair(const GroupStage& s, const Mat& mat, 
                 ti[u][c] = s_im[lane ^ (base[u] ^ urow[c])];
             }
         }
-        d4 k[2] = {}, yr[2], yi[2];
+        d4 yr[2] = {}, yi[2] = {};
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int u = 0; u < 2; u++) k[u] = mfma(ur[c], tr[u][c] + ti[u][c], k[u]);
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            yr[u] = yi[u] = k[u];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                yr[u] = mfma(us[c], -ti[u][c], yr[u]);
-                yi[u] = mfma(ud[c], tr[u][c], yi[u]);
+            for (int u = 0; u < 2; u++) {
+                yr[u] = mfma(ur[c], tr[u][c], yr[u]);
+                yi[u] = mfma(ur[c], ti[u][c], yi[u]);
             }
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                yr[u] = mfma(-ui[c], ti[u][c], yr[u]);
+                yi[u] = mfma(ui[c], tr[u][c], yi[u]);
+            }
+#pragma unroll
+        for (int u = 0; u < 2; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 s_re[lane ^ (base[u] ^ urow[r])] = yr[u][r];
                 s_im[lane ^ (base[u] ^ urow[r])] = yi[u][r];
             }
-        }
     }
 }
 
@@ -189,51 +189,42 @@ __device__ __forceinline__ void stage_unitary5(const GroupStage& s, const Mat& m
     d4 zr[2], zi[2];  // T'[I][0]
 #pragma unroll
     for (int J = 0; J < 2; J++) {
-        d4 xr[2], xi[2], yr[2], yi[2];
-        xr[0] = xr[1] = d4{0, 0, 0, 0};
-#pragma unroll 2
-        for (int K = 0; K < 8; K++) {
-            const uint32_t x = rd ^ group_col_place(group_local(s, 2, 3, K));
-            const double ur = mat(mj + 512 * J + 4 * K);
-#pragma unroll
-            for (int I = 0; I < 2; I++) {
-                const uint32_t xI = I ? x ^ hi_row : x;
-                xr[I] = mfma(s_re[xI] + s_im[xI], ur, xr[I]);
-            }
-        }
-        xi[0] = xr[0];
-        xi[1] = xr[1];
+        d4 p[2] = {}, q[2] = {}, k[2] = {}, xr[2], xi[2], yr[2], yi[2];
 #pragma unroll 2
         for (int K = 0; K < 8; K++) {
             const uint32_t x = rd ^ group_col_place(group_local(s, 2, 3, K));
             const double ur = mat(mj + 512 * J + 4 * K), ui = mat(1024 + mj + 512 * J + 4 * K);
-            const double us = -ur - ui, ud = ui - ur;
 #pragma unroll
             for (int I = 0; I < 2; I++) {
                 const uint32_t xI = I ? x ^ hi_row : x;
-                xr[I] = mfma(s_im[xI], us, xr[I]);
-                xi[I] = mfma(s_re[xI], ud, xi[I]);
+                const double tr = s_re[xI], ti = s_im[xI];
+                p[I] = mfma(tr, ur, p[I]);
+                q[I] = mfma(ti, ui, q[I]);
+                k[I] = mfma(tr + ti, ur + ui, k[I]);
             }
         }
-        yr[0] = yr[1] = d4{0, 0, 0, 0};
 #pragma unroll
-        for (int K = 0; K < 8; K++) {
-            const double xs = xr[K >> 2][K & 3] + xi[K >> 2][K & 3];
-#pragma unroll
-            for (int I = 0; I < 2; I++) yr[I] = mfma(mat(mj + 512 * I + 4 * K), xs, yr[I]);
-            if (K & 1) __builtin_amdgcn_sched_barrier(0);
+        for (int I = 0; I < 2; I++) {
+            xr[I] = p[I] - q[I];
+            xi[I] = k[I] - p[I] - q[I];
+            p[I] = q[I] = k[I] = d4{0, 0, 0, 0};
         }
-        yi[0] = yr[0];
-        yi[1] = yr[1];
 #pragma unroll
         for (int K = 0; K < 8; K++) {
+            const double br = xr[K >> 2][K & 3], bi = xi[K >> 2][K & 3];
 #pragma unroll
             for (int I = 0; I < 2; I++) {
                 const double ur = mat(mj + 512 * I + 4 * K), ui = mat(1024 + mj + 512 * I + 4 * K);
-                yr[I] = mfma(ui - ur, xi[K >> 2][K & 3], yr[I]);
-                yi[I] = mfma(-ur - ui, xr[K >> 2][K & 3], yi[I]);
+                p[I] = mfma(ur, br, p[I]);
+                q[I] = mfma(-ui, bi, q[I]);
+                k[I] = mfma(ur - ui, br + bi, k[I]);
             }
             if (K & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int I = 0; I < 2; I++) {
+            yr[I] = p[I] - q[I];
+            yi[I] = k[I] - p[I] - q[I];
         }
 #pragma unroll
         for (int I = 0; I < 2; I++) {
