@@ -1284,7 +1284,7 @@ std::vector<cd> pair_superoperator(const std::vector<Gate>& circuit, const std::
 // must take the fewest new qubits among the last one on its qubits and those
 // after (a gate on more than two qubits makes a whole-block unitary); then
 // every run of channel-free stages that costs more than one whole-block
-// unitary (24 MFMAs a tile against 16 each) becomes one.
+// unitary (24 MFMAs a tile against 12 each) becomes one.
 void build_stages(const std::vector<Gate>& circuit, const std::vector<int>& gates, int dense,
                   uint32_t qmask, std::vector<FusedStage>& out)
 {
@@ -1328,8 +1328,8 @@ void build_stages(const std::vector<Gate>& circuit, const std::vector<int>& gate
     for (size_t i = 0; i < groups.size();) {
         size_t j = i;
         int cost = 0;
-        while (j < groups.size() && !groups[j].channel) cost += groups[j++].whole ? 24 : 16;
-        if (cost > 24) {
+        while (j < groups.size() && !groups[j].channel) cost += groups[j++].whole ? 2 : 1;
+        if (cost > 2) {
             Group w;
             w.mask = qmask;
             w.whole = true;
