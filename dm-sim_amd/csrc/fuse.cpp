@@ -1380,25 +1380,27 @@ struct StageSpec {
     }
 };
 
-// Channel-free members as unitaries of four bits, each member joining the one
-// that must take the fewest new qubits (as in group_least_growth); then every
-// run of them on five qubits that costs more than one unitary of five bits
-// becomes one.
-std::vector<StageSpec> unitary_stages(const std::vector<Gate>& circuit, const std::vector<int>& gates, int n)
+// Channel-free members as unitaries of four bits, on at most max_k qubits (a wider
+// gate's), each member joining the one that must take the fewest new qubits (as in
+// group_least_growth); then, where max_k allows five, every run of them on five qubits
+// that costs more than one unitary of five bits becomes one.
+std::vector<StageSpec> unitary_stages(const std::vector<Gate>& circuit, const std::vector<int>& gates, int n,
+                                      int max_k)
 {
     std::vector<StageSpec> best;
     double best_cost = 0;
     std::vector<Gate> sub;
     for (int gi : gates) sub.push_back(circuit[gi]);
+    const int kmax = std::min(max_k, 4);
     for (int attempt = 0; attempt < 3; attempt++) {
         std::vector<PB> pbs;
         Seq seq;
         std::vector<long> w;
         if (attempt == 0) {
-            group_least_growth(sub, 4, nullptr, pbs, seq);
+            group_least_growth(sub, kmax, nullptr, pbs, seq);
         } else {
             for (const Gate& g : sub) w.push_back(__builtin_popcount(gate_mask(g)) > 1 ? 100 : attempt == 1 ? 1 : 100);
-            group_frontier(sub, n, 4, false, true, nullptr, pbs, seq, &w);
+            group_frontier(sub, n, kmax, false, true, nullptr, pbs, seq, &w);
         }
         std::vector<StageSpec> out;
         for (const PB& pb : pbs) {
@@ -1406,7 +1408,7 @@ std::vector<StageSpec> unitary_stages(const std::vector<Gate>& circuit, const st
             for (int i : pb.gates) sp.members.push_back(gates[i]);
             out.push_back(std::move(sp));
         }
-        for (size_t i = 0; i < out.size(); i++) {
+        for (size_t i = 0; i < out.size() && max_k > 4; i++) {
             uint32_t mask = 0;
             double cost = 0;
             size_t take = i;
@@ -1439,10 +1441,10 @@ std::vector<StageSpec> unitary_stages(const std::vector<Gate>& circuit, const st
 // member joining the one that must take the fewest new qubits; then each run of
 // channel-free ones becomes unitary_stages where those cost less.
 std::vector<StageSpec> group_stages(const std::vector<Gate>& circuit, const std::vector<int>& gates,
-                                    int dense, int n)
+                                    int dense, int n, int max_k)
 {
     const std::vector<int> matrix(gates.begin(), gates.begin() + dense);
-    if (!has_channel(circuit, gates, dense)) return unitary_stages(circuit, matrix, n);
+    if (!has_channel(circuit, gates, dense)) return unitary_stages(circuit, matrix, n, max_k);
     std::vector<StageSpec> pairs;
     std::vector<char> noisy;
     for (int gi : matrix) {
@@ -1456,8 +1458,10 @@ std::vector<StageSpec> group_stages(const std::vector<Gate>& circuit, const std:
             }
         int best = -1, best_g = 99;
         for (int b = first; b < (int)pairs.size() && width <= 2; b++) {
-            const int grow = __builtin_popcount(pairs[b].mask | S) - __builtin_popcount(pairs[b].mask);
-            if (pairs[b].kind == GS_PAIR && __builtin_popcount(pairs[b].mask | S) <= 2 && grow <= best_g) {
+            const int have = __builtin_popcount(pairs[b].mask), with = __builtin_popcount(pairs[b].mask | S);
+            const int grow = with - have;
+            if (pairs[b].kind == GS_PAIR && with <= 2 && with <= std::max({max_k, width, have}) &&
+                grow <= best_g) {
                 best = b;
                 best_g = grow;
             }
@@ -1480,7 +1484,7 @@ std::vector<StageSpec> group_stages(const std::vector<Gate>& circuit, const std:
             run.insert(run.end(), pairs[j].members.begin(), pairs[j].members.end());
             cost += pairs[j].cost();
         }
-        const std::vector<StageSpec> u = unitary_stages(circuit, run, n);
+        const std::vector<StageSpec> u = unitary_stages(circuit, run, n, max_k);
         for (const StageSpec& s : u) as_unitary += s.cost();
         if (as_unitary < cost) {
             out.insert(out.end(), u.begin(), u.end());
@@ -2184,7 +2188,7 @@ double group_us(double base, double stage_cost)
 // structural scores; with one, the cheapest of that and four other scorings
 // (one-qubit gates weighing 400, 100 and 30, and the gates' predicted unfused
 // times), each searched on a host thread of its own.
-int choose_groups(const std::vector<Gate>& circuit, const std::vector<Gate>& todo, int n,
+int choose_groups(const std::vector<Gate>& circuit, const std::vector<Gate>& todo, int n, int max_k,
                   const Units* units, CostModel* model, std::vector<PB>& pbs, Seq& seq, PlanInfo& pi)
 {
     constexpr int kCands = 5;
@@ -2224,7 +2228,7 @@ int choose_groups(const std::vector<Gate>& circuit, const std::vector<Gate>& tod
                 if (!model) continue;
                 const int dense = pb.dense < 0 ? (int)pb.gates.size() : pb.dense;
                 double cost = 0;
-                for (const StageSpec& sp : group_stages(circuit, pb.gates, dense, n)) cost += sp.cost();
+                for (const StageSpec& sp : group_stages(circuit, pb.gates, dense, n, max_k)) cost += sp.cost();
                 us[c] += group_us(base, cost);
             }
         } catch (...) {
@@ -2254,10 +2258,10 @@ int choose_groups(const std::vector<Gate>& circuit, const std::vector<Gate>& tod
 }
 
 // The plan of a circuit as group sweeps (six qubits each, stages of at most
-// four, or five for a gate that wide) and a relabelling home at the end.
+// max_k, or as wide as a gate) and a relabelling home at the end.
 // Each sweep is written with its qubits (after its trailing index map) on bits
 // 0..5, those that the next sweep shares lowest.
-int build_group_plan(const std::vector<Gate>& circuit, int n, CostModel* model, FusedPlan** out,
+int build_group_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model, FusedPlan** out,
                      PlanInfo* info)
 {
     PlanInfo pi;
@@ -2268,7 +2272,7 @@ int build_group_plan(const std::vector<Gate>& circuit, int n, CostModel* model, 
     const std::vector<Gate>& todo = channels ? units->gates : circuit;
     std::vector<PB> pbs;
     Seq seq;
-    int rc = choose_groups(circuit, todo, n, units.get(), model, pbs, seq, pi);
+    int rc = choose_groups(circuit, todo, n, max_k, units.get(), model, pbs, seq, pi);
     if (rc) return rc;
     std::unique_ptr<Plan> plan(new Plan());
     plan->n = n;
@@ -2295,7 +2299,7 @@ int build_group_plan(const std::vector<Gate>& circuit, int n, CostModel* model, 
             return (uint32_t)__builtin_popcount(b.qmask & ((1u << bo.sigma[q]) - 1u));
         };
         const int dense = pb.dense < 0 ? (int)pb.gates.size() : pb.dense;
-        for (const StageSpec& sp : group_stages(circuit, pb.gates, dense, n)) {
+        for (const StageSpec& sp : group_stages(circuit, pb.gates, dense, n, max_k)) {
             GroupStage st;
             std::memset(&st, 0, sizeof(st));
             st.kind = sp.kind;
@@ -2418,7 +2422,7 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
         if (linear) {
             PlanInfo gi, ai;
             FusedPlan *grouped = nullptr, *alone = nullptr;
-            int rc = build_group_plan(circuit, n, tile_bits > 0 ? nullptr : model, &grouped, &gi);
+            int rc = build_group_plan(circuit, n, max_k, tile_bits > 0 ? nullptr : model, &grouped, &gi);
             if (rc) return rc;
             bool channels = false;
             for (const Gate& g : circuit) channels = channels || g.op == OP_KRAUS;

@@ -176,8 +176,8 @@ inline bool permuting_pays(int n, double sweeps, double permuting, double sweeps
 // block's output lands in aligned 16-column runs; rho returns to the
 // circuit's bit order (k_relabel) before any other step and at the end.
 // group (with herm and fold): the whole plan as group sweeps (k_group) of six
-// qubits whose stages are the blocks: several blocks of at most four qubits
-// (five for a five-qubit gate or where it costs less) to a sweep.
+// qubits whose stages are the blocks: several blocks of at most max_k qubits
+// (five for a five-qubit gate) to a sweep.
 // resident (where resident_wanted, with allow_perm): the blocks run on resident
 // rows; the model's prices still are those of sweeps.
 int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostModel* model,

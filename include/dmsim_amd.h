@@ -150,7 +150,11 @@ int dmx_dump(const dmx_sim* sim, char* buf, size_t cap, size_t* needed);
 int dmx_set_method(dmx_sim* sim, int method);
 
 /* Fusion limit for DMX_METHOD_FUSED: blocks grow to at most k qubits (1..5,
- * default 4); a gate on five qubits always forms a five-qubit block. */
+ * default 4); a gate on five qubits always forms a five-qubit block.  Circuits
+ * with noise channels: from 7 qubits channels run inside blocks of at most
+ * min(k, 4) qubits (with a gate on five, between blocks); from 12, and from 13
+ * qubits where a gate is on five, several blocks of at most k qubits run in
+ * one sweep on six, unless permuting blocks or Hermitian sweeps are off. */
 int dmx_set_fusion_max_k(dmx_sim* sim, uint32_t k);
 
 /* Extension with no counterpart in the reference: whether four-qubit blocks of
