@@ -1824,14 +1824,15 @@ int choose_grouping(const std::vector<Gate>& circuit, int n, int kmax, bool allo
 }
 
 // Learned choice per block: fused at tile width m (4..min(8, n)) or its
-// member gates' primitive sweeps on both indices.  Sets blocks[b].m, fills
-// plain[b] with the primitives of blocks that run unfused.
+// member gates' primitive sweeps on both indices (not fused_only).  Sets blocks[b].m,
+// fills plain[b] with the primitives of blocks that run unfused.
 // A candidate replaces the default only if predicted at least this much faster
 // (the model's median error on held-out launches is about 10 %).
 constexpr double kMargin = 0.92;
 
 int choose_executions(const std::vector<Gate>& circuit, int n, BlockPlan& bp, CostModel& model,
-                      std::vector<std::vector<PrimOp>>& plain, PlanInfo& info, bool herm)
+                      std::vector<std::vector<PrimOp>>& plain, PlanInfo& info, bool herm,
+                      bool fused_only = false)
 {
     const int nb = (int)bp.blocks.size();
     // Hermitian plans: one fused option per block, the Hermitian sweep at width
@@ -1874,7 +1875,7 @@ int choose_executions(const std::vector<Gate>& circuit, int n, BlockPlan& bp, Co
             feats.emplace_back(f, f + kMlpFeatures);
         }
         std::vector<PrimOp> ps;
-        bool ok = true;
+        bool ok = !fused_only;
         for (int gi : bp.members[b])
             ok = ok && circuit[gi].op != OP_KRAUS && lower_gate(circuit[gi], ps);
         if (!ok) continue;
@@ -2468,12 +2469,10 @@ int build_fused_plan(const std::vector<Gate>& circuit, int n, int max_k, CostMod
         for (FusedBlock5& fb : bp.blocks5)
             if (tile_bits5_ok(n, tile_bits, fb.qmask)) fb.m = (uint32_t)tile_bits;
     } else if (model) {
-        rc = choose_executions(circuit, n, bp, *model, plain, pi, herm);
+        rc = choose_executions(circuit, n, bp, *model, plain, pi, herm, resident);
         if (rc) return rc;
         rc = choose_fused5(circuit, n, bp, *model, sub, pi);
         if (rc) return rc;
-        if (resident)  // no block as primitive sweeps, whatever these would take
-            for (auto& p : plain) p.clear();
     }
     Plan* plan = new Plan();
     plan->n = n;

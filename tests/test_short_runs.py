@@ -191,3 +191,31 @@ def test_batched_short_circuits_equal_single_runs():
                 got = b.get_dm(i)
                 assert np.array_equal(got[0], re) and np.array_equal(got[1], im), i
         b.close()
+
+
+@pytest.mark.parametrize("n", [9, 11])
+def test_plan_info_counts_resident_blocks_once(n):
+    """With a cost model, a block of one cheap gate counts as the fused block it runs as, and
+    the predicted time is that of the blocks as fused sweeps."""
+    import costdata
+    import dmsim_amd as dm
+    model = costdata.default_model()
+    t = W.GateTable(n)
+    for a in (0, 4):
+        for g in W.random_mixed(4, 40, 3 + a, gate_set=["U3", "CX"]).qbs:
+            t.add("U3", [a + g[0]], (0.3, 0.2, 0.1)) if g[0] == g[1] or g[1] >= 4 else \
+                t.add("RYY", [a + g[0], a + g[1]], (0.4,))
+    t.add("T", [8])
+    s = dm.Sim(n)
+    s.set_method(dm.METHOD_FUSED)
+    s.set_cost_model(model)
+    s.append_table(t)
+    s.upload()
+    s.set_profiling(True)
+    s.run()
+    assert s.profile()["k_resident"]["calls"] == 2
+    info = s.plan_info()
+    print(info, flush=True)
+    assert info["plain_blocks"] == 0 and info["fused_blocks"] == 3
+    assert sum(info["tiles"].values()) == info["fused_blocks"]
+    model.close()
