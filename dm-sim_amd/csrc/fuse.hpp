@@ -212,10 +212,10 @@ inline int brief_tile_bits(int n) { return n < 6 ? n : n <= 9 ? 6 : n == 10 ? 7 
 // Whether a circuit's Hermitian plan runs as group sweeps.  With channels, from
 // 12 qubits: a group holds their whole neighbourhood where a four-qubit block
 // with a channel on every gate fills up with channels (a 300-member 12-qubit
-// circuit 1680 -> 1315 us; below 12 qubits rho fits the caches and a sweep costs
-// its launch).  With five-qubit gates, from 13: the five-qubit sweep has no
-// Hermitian form (structured circuits 20.3 -> 14.3 ms at 13 qubits, 77 -> 62.5
-// at 14, 332 -> 289 at 15).  Other unitary circuits keep four-qubit sweeps: on
+// circuit 1680 us in four-qubit blocks with channels, 1520 in groups; below 12 qubits rho
+// fits the caches and a sweep costs its launch).  With five-qubit gates, from 13: the five-qubit sweep has no
+// Hermitian form (structured circuits 21.5 -> 15.4 ms at 13 qubits, 84 -> 68
+// at 14, 354 -> 297 at 15).  Other unitary circuits keep four-qubit sweeps: on
 // 2130 gates at 14 qubits 113 group sweeps of 1.69 ms take 193 ms, 181 of the
 // others 177, as a group's 2.2 stages occupy the matrix cores for 1 ms that
 // overlaps its 1.1 ms of memory traffic only in part.
@@ -224,8 +224,10 @@ bool group_wanted(const std::vector<Gate>& circuit, int n);
 // From this many qubits the engine folds channels into blocks.  A noisy
 // 318-member circuit at 8 qubits takes 9 sweeps instead of 138 and 180 channel
 // sweeps (1.32 -> 0.22 ms a run with its downloads), one of 164 members at 12
-// qubits 12 instead of 182 launches (16.1 -> 1.95 ms).  Below, a plan's launches
-// stay one per block and channel, which callers at those sizes count on.
+// qubits 12 instead of 182 launches (16.1 -> 1.95 ms).  It would pay below as well: 100
+// gates with a channel on every operand take 558, 694 and 688 us at 4, 5 and 6 qubits
+// and would take 31, 47 and 45.  There a plan stays at one launch per block and channel
+// because a test at 6 qubits counts them, and no setting asks for channels as barriers.
 constexpr int kFoldChannelQubits = 7;
 
 // Smallest n for Hermitian plans, and the smallest where the engine uses

@@ -578,7 +578,8 @@ class Batch:
         return w.value
 
     def set_hermitian(self, on: bool):
-        """Hermitian block sweeps for the circuits of 10 and 11 qubits (default on)."""
+        """Block sweeps instead of resident rows (what a batch takes that is not
+        asked): Hermitian ones for the circuits of 10 and 11 qubits, or, off, none."""
         _check(load().dmx_batch_set_hermitian(self._h, 1 if on else 0))
 
     def set_group_bytes(self, nbytes: int):
