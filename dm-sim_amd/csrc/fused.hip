@@ -836,10 +836,10 @@ hipError_t launch_fused4_herm(const double* re, const double* im, double* re_out
     // A multiple of 128 workgroups (herm_slot): 16 per XCD group.  Two per CU run
     // at a time and each begins with a few us of index-map set-up, so no more
     // than that while a workgroup has a dozen items or so at most (us a sweep,
-    // 512 against 4096 workgroups: 12 qubits, 2176 items, 82 against 112; 13
-    // qubits, 8448, 265 against 308); at 14 qubits (33280 items) twice as many,
-    // which even out the last wave (980 against 1000 with 512, 1006 with 4096);
-    // above, the set-up is lost in the sweep and the launch deals best
+    // 512 against 4096 workgroups: 12 qubits, 2176 items, 86 against 117; 13
+    // qubits, 8448, 256 against 307); at 14 qubits (33280 items) twice as many, which is
+    // as good as any (954 against 1006 with 512 and 994 with 4096, where runs differ by
+    // 4 %); above, the set-up is lost in the sweep and the launch deals best
     // (15 qubits: a run of 76 steps 330 ms with 4096 against 342 with 1024).
     const uint64_t fit = items < 16384 ? 512 : items < 65536 ? 1024 : ~0ull;
     const uint64_t cap = fit < (uint64_t)max_blocks ? fit : (uint64_t)max_blocks;

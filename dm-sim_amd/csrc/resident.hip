@@ -11,15 +11,15 @@
 // (none where a wave holds the row, up to 8 qubits).  Index permutations between
 // blocks (X, CX, SWAP) only change the places that later records name.
 //
-// Bound: up to 9 qubits one wave's chain of LDS reads, 12 MFMAs and LDS writes (0.64
+// Bound: up to 9 qubits one wave's chain of LDS reads, 12 MFMAs and LDS writes (0.63
 // us a block and pass at n = 8, where 256 waves have a SIMD each); from 10 the FP64
-// matrix cores, busy 64 % of the time at n = 11 with eight waves of a tile each (9.1
-// us a block and pass for 6.2 at 65 TFLOP/s; LDS 19 % of the time, 15 % of that
-// bank conflicts).  There four waves of two tiles, one after the other, leave
-// registers for five workgroups a CU instead of two: 601 gates 665 -> 638 us a pass,
-// 96 circuits of 6 to 11 qubits 16.4 -> 14.9 ms.
-// Against one launch per block: 90 blocks at n = 8 586 -> 117 us a run, 30 at n = 11
-// 1305 -> 560.
+// matrix cores, busy 69 % of the time at n = 11 (8.3 us a block and pass for 6.2 at 65
+// TFLOP/s; LDS 21 % of the time, 15 % of that bank conflicts), with four waves of two
+// tiles, one after the other, which leave registers for five workgroups a CU: with eight
+// waves of a tile, two workgroups, 64 % (601 gates 665 -> 638 us a pass, 96 circuits of
+// 6 to 11 qubits 16.4 -> 14.9 ms).
+// Against one launch per block: 90 blocks at n = 8 586 -> 113 us a run, 30 at n = 11
+// 1305 -> 520.
 #include <hip/hip_runtime.h>
 
 #include "resident.hpp"

@@ -8,7 +8,7 @@
 // in-place conjugate transpose and this kernel again.
 //
 // Bound: from 10 qubits the FP64 VALU (mul and add apart, as the reference
-// rounds them: 64-68 % busy at n = 13) and, between groups of primitives on at
+// rounds them: 77-78 % busy at n = 11 and 13) and, between groups of primitives on at
 // most K target bits, one LDS round trip of the row; below, the latency of one
 // wave's chain of steps (0.3 us each: dispatch, a few dependent FP64
 // operations and a third of an LDS round trip).

@@ -43,7 +43,8 @@ enum dmx_op {
 };
 
 /* Execution methods (dmx_set_method). */
-#define DMX_METHOD_PLAIN 0        /* gate by gate, whole rows of rho on chip (n <= 14)           */
+#define DMX_METHOD_PLAIN 0        /* gate by gate, whole rows of rho on chip (n <= 14; short
+                                     stretches between channels as PLAIN_LAUNCH, same bits)  */
 #define DMX_METHOD_PLAIN_LAUNCH 1 /* gate by gate, 2 sweeps and launches per primitive           */
 #define DMX_METHOD_FUSED 2        /* gates fused into dense 4- and 5-qubit blocks, one sweep each */
 
@@ -177,7 +178,9 @@ int dmx_set_fusion_permute(dmx_sim* sim, uint32_t on);
  *
  * With mode 1, permuting blocks on, no fixed tile width and blocks of at most
  * four qubits, unitary circuits of 4 to 11 qubits make no sweeps: all blocks run
- * in two launches that hold whole rows of rho on chip. */
+ * in two launches that hold whole rows of rho on chip (with a conjugate
+ * transpose between them from 10 qubits).  One or two blocks without a
+ * trailing permutation run as sweeps in place, from 5 qubits. */
 int dmx_set_fusion_hermitian(dmx_sim* sim, uint32_t mode);
 
 /* Extension: the greedy plan's tile width measured (on = 1, default): without
@@ -381,7 +384,12 @@ int dmx_batch_run(dmx_batch* b);
 /* E_c = sum of weight * Re Tr(P rho_c) per circuit, out[circuit count]. */
 int dmx_batch_energies(dmx_batch* b, double* out);
 
-/* rho of circuit id after the last run, dmx_get_dm's convention (4^n doubles each). */
+/* rho of circuit id after the last run, dmx_get_dm's convention (4^n doubles
+ * each).  Where a circuit of 10 or 11 qubits runs on rows held on chip (the
+ * default, see dmx_batch_set_hermitian) its planes are handed out as they lie
+ * then, conj-transposed: rho is Hermitian, so the entries are dmx_get_dm's to
+ * rounding, and bit for bit the conjugate transpose of what the circuit's own
+ * run returns.  All other circuits' are bit for bit their own run's. */
 int dmx_batch_get_dm(dmx_batch* b, uint32_t id, double* re, double* im);
 
 /* Device time of the last run, launches per run, circuits, total API gates. */
@@ -430,7 +438,8 @@ int dmx_batch_set_group_bytes(dmx_batch* b, uint64_t bytes);
 
 /* Extension: the batched circuits' blocks as sweeps, which a batch that this is
  * not called for runs on resident rows instead (all blocks of a circuit in two
- * launches that hold whole rows of rho on chip).  On: Hermitian block sweeps
+ * launches that hold whole rows of rho on chip; one or two blocks in place, as
+ * dmx_upload runs the circuit alone).  On: Hermitian block sweeps
  * for the circuits of 10 and 11 qubits (below 10 in-order blocks are faster in a
  * batch): their blocks run as batched Hermitian sweeps (the tiles
  * on and above the diagonal, each result written with its conjugate
