@@ -178,9 +178,15 @@ struct Plan : FusedPlan {
                        PlanInfo& info) override
     {
         *chosen = 0;
+        // Blocks with channels take two to five times as long and there are few of them:
+        // a sample half as large, timed twice instead of three times (upload of an ansatz
+        // with a channel on every operand: 318 members at 8 qubits 2.76 -> 1.64 ms, 444
+        // at 11 16.3 -> 6.6; runs at the widths chosen are within 1 %).
+        const size_t most = channels_inside ? 4 : 8;
+        const int reps = channels_inside ? 2 : 3;
         std::vector<int> sample;
         for (const Step& st : steps)
-            if (st.type == ST_FUSED4 && sample.size() < 8) sample.push_back(st.index);
+            if (st.type == ST_FUSED4 && sample.size() < most) sample.push_back(st.index);
         if (sample.empty()) return DMX_OK;
         bool all_q0 = true;
         for (int b : sample) all_q0 = all_q0 && (blocks[b].qmask & 1u);
@@ -190,7 +196,7 @@ struct Plan : FusedPlan {
         int best_m = 0;
         float best_ms = 0.f;
         for (int m = all_q0 ? 4 : 5; m <= std::min(8, nq) && e == hipSuccess; m++) {
-            for (int rep = 0; rep < 4 && e == hipSuccess; rep++) {  // rep 0 warms up
+            for (int rep = 0; rep <= reps && e == hipSuccess; rep++) {  // rep 0 warms up
                 if (rep == 1) e = hipEventRecord(e0, stream);
                 for (int b : sample)
                     if (e == hipSuccess)
